@@ -12,7 +12,9 @@
 // Kernels:
 //   deltanet_project_kernel   grid ceil(R/16): 16 rows of the concatenated
 //                             [qkv | z | a | b] weight space per workgroup,
-//                             streamed once and applied to every token.
+//                             streamed once and applied to every token; batches
+//                             of kGemmMinTokens or more at the shapes norm_gemm_ok
+//                             takes run token_gemm_kernel (fk_gemm.hip) instead.
 //   deltanet_conv_kernel      one thread per channel, sliding window in registers.
 //   deltanet_recurrent_kernel grid (Hv, ceil(D/32)); a workgroup owns a
 //                             D x 32 fp32 state tile in registers (16 rows per
@@ -73,6 +75,10 @@ struct ProjArgs {
 };
 
 constexpr int kProjMaxFusedTokens = 64;
+// From this many tokens the projections run on the matrix cores
+// (launch_norm_gemm): 25-26 us at 3 to 32 tokens where this kernel takes 24.0
+// us at 2, 29.8 at 4 and 41.6 at 8 (the model's 12,352 rows).
+constexpr int kGemmMinTokens = 4;
 
 template <bool BFW, bool BFX, int NJ>
 __global__ __launch_bounds__(256) void deltanet_project_kernel(ProjArgs a) {
@@ -1491,6 +1497,8 @@ __global__ __launch_bounds__(512) void deltanet_step_kernel(StepArgs a) {
 // Host launchers
 // ---------------------------------------------------------------------------
 static int launch_project(const ProjArgs& pa, int weight_dtype, int hidden_dtype, hipStream_t s) {
+  if (!pa.conv_out && pa.T >= kGemmMinTokens && norm_gemm_ok(pa.rows, pa.H, weight_dtype, pa.nw_dt))
+    return launch_norm_gemm(pa.x, hidden_dtype, pa.nw, pa.w, pa.rows, pa.out, pa.T, pa.H, pa.eps, pa.off, s);
   const int R = pa.rows[0] + pa.rows[1] + pa.rows[2] + pa.rows[3];
   const int grid = (R + kProjRows - 1) / kProjRows;
   const bool bfw = weight_dtype == FK_DTYPE_BF16, bfx = hidden_dtype == FK_DTYPE_BF16, wide = pa.H > 2048;

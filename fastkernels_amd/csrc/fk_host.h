@@ -33,6 +33,13 @@ int launch_norm_projection(const void* x, int x_dt, const void* nw, int nw_dt, c
                            const int (&rows)[4], float* const (&out)[4], int weight_dt, int T, int H, float eps,
                            float off, hipStream_t s);
 
+// Token-batch projections on the matrix cores (fk_gemm.hip), for up to four
+// bf16 matrices of a multiple of 16 rows each, K a multiple of 64 and a bf16
+// norm weight: out[i] = RMSNorm(x) * (off + nw) . w[i]^T, f32 [T, rows[i]].
+bool norm_gemm_ok(const int (&rows)[4], int K, int weight_dt, int nw_dt);
+int launch_norm_gemm(const void* x, int x_dt, const void* nw, const void* const (&w)[4], const int (&rows)[4],
+                     float* const (&out)[4], int T, int K, float eps, float off, hipStream_t s);
+
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 inline bool is_float_dtype(int dt) { return dt == FK_DTYPE_F32 || dt == FK_DTYPE_BF16; }
