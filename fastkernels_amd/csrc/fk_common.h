@@ -87,6 +87,26 @@ __device__ __forceinline__ void split_hi_lo8(const float (&v)[8], u32x4& hi, u32
   lo = u32x4{l[0], l[1], l[2], l[3]};
 }
 
+// fp32 values as three bf16 terms each, hi = bf16(v), mid = bf16(v - hi),
+// lo = bf16(v - hi - mid) (round to nearest even): all 24 bits of v as MFMA
+// operands.  Packed in pairs.  A value whose hi term is infinite or NaN has no
+// remainder (inf - inf would turn it to NaN).
+__device__ __forceinline__ void split3_2(float a, float b, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
+  hi = pack_bf16x2(a, b);
+  const float ha = __uint_as_float(hi << 16), hb = __uint_as_float(hi & 0xffff0000u);
+  const float ra = fabsf(ha) < INFINITY ? a - ha : 0.f, rb = fabsf(hb) < INFINITY ? b - hb : 0.f;
+  mid = pack_bf16x2(ra, rb);
+  lo = pack_bf16x2(ra - __uint_as_float(mid << 16), rb - __uint_as_float(mid & 0xffff0000u));
+}
+__device__ __forceinline__ void split3_8(const float (&v)[8], u32x4& hi, u32x4& mid, u32x4& lo) {
+  uint32_t h[4], m[4], l[4];
+#pragma unroll
+  for (int p = 0; p < 4; ++p) split3_2(v[2 * p], v[2 * p + 1], h[p], m[p], l[p]);
+  hi = u32x4{h[0], h[1], h[2], h[3]};
+  mid = u32x4{m[0], m[1], m[2], m[3]};
+  lo = u32x4{l[0], l[1], l[2], l[3]};
+}
+
 template <bool BF16>
 __device__ __forceinline__ Raw8<BF16> load_raw8(const void* base, size_t elem_index) {
   Raw8<BF16> r;

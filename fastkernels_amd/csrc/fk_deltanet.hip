@@ -41,8 +41,18 @@ constexpr int kOutRows = 8;     // W_out rows per workgroup (2 per wave)
 struct DnWs {
   uint32_t* tickets;  // [Hv]
   float* core;        // [T, Hv*D] raw recurrent output
-  float* normed;      // [T, Hv*D] gated-RMSNorm output
+  float* normed;      // [T, Hv*D] gated-RMSNorm output, or
+  uint16_t* planes;   // [3][T][Hv*D] the same as three bf16 terms (split3_2)
+  float* part;        // partial sums of the output projection
+  size_t part_bytes;
 };
+
+// Partial sums of the output projection for 2,048 output rows: up to 8 splits
+// of K, fewer as the tokens fill the chip by themselves (launch_plane_gemm).
+static size_t dn_part_bytes(int T) {
+  const size_t splits = T >= 1024 ? 1 : T <= 128 ? 8 : (size_t)(1024 / T);
+  return splits > 1 ? splits * (size_t)T * 2048 * 4 : 0;
+}
 
 static size_t dn_ws_layout(int T, int Hv, int D, char* base, DnWs* ws) {
   size_t off = 0;
@@ -53,7 +63,10 @@ static size_t dn_ws_layout(int T, int Hv, int D, char* base, DnWs* ws) {
   };
   ws->tickets = reinterpret_cast<uint32_t*>(take((size_t)Hv * 4));
   ws->core = reinterpret_cast<float*>(take((size_t)T * Hv * D * 4));
-  ws->normed = reinterpret_cast<float*>(take((size_t)T * Hv * D * 4));
+  ws->planes = reinterpret_cast<uint16_t*>(take((size_t)T * Hv * D * 6));
+  ws->normed = reinterpret_cast<float*>(ws->planes);
+  ws->part_bytes = dn_part_bytes(T);
+  ws->part = reinterpret_cast<float*>(take(ws->part_bytes));
   return off;
 }
 
@@ -84,6 +97,11 @@ constexpr int kProjMaxFusedTokens = 64;
 // (launch_norm_gemm): 25-26 us at 3 to 32 tokens where this kernel takes 24.0
 // us at 2, 29.8 at 4 and 41.6 at 8 (the model's 12,352 rows).
 constexpr int kGemmMinTokens = 4;
+// From this many tokens the recurrence runs as the scan and the output
+// projection on the matrix cores, two to three more launches: the operator
+// takes 28 us from 3 to 32 tokens where the two kernels before took 24.5 us at
+// 1 and 2 (host-bound there), 30 at 3, 57 at 8 and 192 at 32.
+constexpr int kScanMinTokens = 3;
 
 template <bool BFW, bool BFX, int NJ>
 __global__ __launch_bounds__(256) void deltanet_project_kernel(ProjArgs a) {
@@ -252,19 +270,22 @@ struct ConvArgs {
   const void* w;
   int w_dt;
   int T, C, KS;
+  int rows;  // rows per thread
   float* out;
   void* next_state;
 };
 
-// Thread (channel, block of kConvTokens rows): the window in registers, its
-// first KS - 1 inputs read again from the rows (or the state) before the
-// block.  One thread per channel for every row was a serial chain of loads on
-// 32 workgroups (0.39 us a row: 198 us at 512 rows, 8,192 channels; now 12).
+// Thread (channel, block of `rows` rows): the window in registers, its first
+// KS - 1 inputs read again from the rows (or the state) before the block.
+// One thread per channel for every row was a serial chain of loads on 32
+// workgroups (0.39 us a row: 198 us at 512 rows, 8,192 channels; in blocks of
+// 8 rows 12).  Outputs written over the inputs (or the state in place) keep
+// one block of all rows, where a thread reads what it overwrites first.
 constexpr int kConvTokens = 8;
 __global__ __launch_bounds__(256) void deltanet_conv_kernel(ConvArgs a) {
   const int c = blockIdx.x * 256 + threadIdx.x;
   if (c >= a.C) return;
-  const int t0 = blockIdx.y * kConvTokens, nt = min(kConvTokens, a.T - t0);
+  const int t0 = blockIdx.y * a.rows, t1 = min(t0 + a.rows, a.T);
   float win[8];
   float wk[8];
 #pragma unroll
@@ -275,29 +296,46 @@ __global__ __launch_bounds__(256) void deltanet_conv_kernel(ConvArgs a) {
                        : load_scalar(a.mixed, a.mixed_dt, (size_t)u * a.C + c);
     wk[j] = j < a.KS ? load_scalar(a.w, a.w_dt, (size_t)c * a.KS + j) : 0.f;
   }
-  float in[kConvTokens];
+  for (int tb = t0; tb < t1; tb += kConvTokens) {
+    float in[kConvTokens];
 #pragma unroll
-  for (int i = 0; i < kConvTokens; ++i)
-    in[i] = load_scalar(a.mixed, a.mixed_dt, (size_t)(t0 + min(i, nt - 1)) * a.C + c);
+    for (int i = 0; i < kConvTokens; ++i)
+      in[i] = load_scalar(a.mixed, a.mixed_dt, (size_t)min(tb + i, t1 - 1) * a.C + c);
 #pragma unroll
-  for (int i = 0; i < kConvTokens; ++i) {
-    if (i >= nt) break;
+    for (int i = 0; i < kConvTokens; ++i) {
+      if (tb + i >= t1) break;
 #pragma unroll
-    for (int j = 0; j < 7; ++j)
-      if (j + 1 < a.KS) win[j] = win[j + 1];
+      for (int j = 0; j < 7; ++j)
+        if (j + 1 < a.KS) win[j] = win[j + 1];
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      if (j == a.KS - 1) win[j] = in[i];
-    float acc = 0.f;
+      for (int j = 0; j < 8; ++j)
+        if (j == a.KS - 1) win[j] = in[i];
+      float acc = 0.f;
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      if (j < a.KS) acc = fmaf(wk[j], win[j], acc);
-    a.out[(size_t)(t0 + i) * a.C + c] = silu(acc);
+      for (int j = 0; j < 8; ++j)
+        if (j < a.KS) acc = fmaf(wk[j], win[j], acc);
+      a.out[(size_t)(tb + i) * a.C + c] = silu(acc);
+    }
   }
-  if (t0 + nt < a.T) return;
+  if (t1 < a.T) return;
 #pragma unroll
   for (int j = 0; j < 8; ++j)
     if (j < a.KS) store_scalar(a.next_state, a.state_dt, (size_t)c * a.KS + j, win[j]);
+}
+
+static bool ranges_overlap(const void* p, size_t np, const void* q, size_t nq) {
+  const uintptr_t a = reinterpret_cast<uintptr_t>(p), b = reinterpret_cast<uintptr_t>(q);
+  return a < b + nq && b < a + np;
+}
+
+static int launch_conv(ConvArgs ca, hipStream_t s) {
+  const size_t n = (size_t)ca.T * ca.C, ns = (size_t)ca.C * ca.KS * (ca.state_dt == FK_DTYPE_BF16 ? 2 : 4);
+  const bool in_place = ranges_overlap(ca.mixed, n * (ca.mixed_dt == FK_DTYPE_BF16 ? 2 : 4), ca.out, n * 4) ||
+                        ranges_overlap(ca.state, ns, ca.next_state, ns);
+  ca.rows = in_place ? ca.T : kConvTokens;
+  const dim3 grid((unsigned)((ca.C + 255) / 256), (unsigned)((ca.T + ca.rows - 1) / ca.rows));
+  hipLaunchKernelGGL(deltanet_conv_kernel, grid, dim3(256), 0, s, ca);
+  return check_launch("deltanet_conv_kernel");
 }
 
 // ---------------------------------------------------------------------------
@@ -612,7 +650,9 @@ __global__ __launch_bounds__(256) void deltanet_scan_kernel(RecArgs a) {
     store_scalar(a.next_state, a.dt[4], sbase + (size_t)((i >> 2) * 64 + sub * 4 + (i & 3)) * D, S[i]);
 }
 
-// Gated RMSNorm of the scan's outputs: a wavefront per (token, head) of 128.
+// Gated RMSNorm of the scan's outputs, a wavefront per (token, head) of 128:
+// as fp32, or as the bf16 planes that launch_plane_gemm reads (PLANES).
+template <bool PLANES>
 __global__ __launch_bounds__(256) void deltanet_gate_kernel(RecArgs a) {
   constexpr int D = 128;
   const int lane = threadIdx.x & 63;
@@ -623,7 +663,16 @@ __global__ __launch_bounds__(256) void deltanet_gate_kernel(RecArgs a) {
   const float z0 = load_scalar(a.z, a.dt[1], i), z1 = load_scalar(a.z, a.dt[1], i + 1);
   const float w0 = load_scalar(a.lnw, a.dt[6], lane * 2), w1 = load_scalar(a.lnw, a.dt[6], lane * 2 + 1);
   const float rs = rsqrtf(wave_sum(fmaf(o.x, o.x, o.y * o.y)) / (float)D + a.eps);
-  *reinterpret_cast<float2*>(a.ws.normed + i) = make_float2(o.x * rs * w0 * silu(z0), o.y * rs * w1 * silu(z1));
+  const float2 v = make_float2(o.x * rs * w0 * silu(z0), o.y * rs * w1 * silu(z1));
+  if constexpr (PLANES) {
+    uint32_t t[3];
+    split3_2(v.x, v.y, t[0], t[1], t[2]);
+    const size_t plane = (size_t)a.T * a.Hv * D;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) *reinterpret_cast<uint32_t*>(a.ws.planes + q * plane + i) = t[q];
+  } else {
+    *reinterpret_cast<float2*>(a.ws.normed + i) = v;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1724,12 +1773,19 @@ static int launch_recurrent_output(const RecArgs& ra, const void* out_proj_weigh
                                    float* residual_out, hipStream_t s) {
   int st;
   // (the scan reads q and k rows of f32 sixteen bytes at a time)
-  if (ra.D == 128 && ra.dt[0] == FK_DTYPE_F32 && aligned16(ra.mixed)) {
+  if (ra.T >= kScanMinTokens && ra.D == 128 && ra.dt[0] == FK_DTYPE_F32 && aligned16(ra.mixed)) {
     hipLaunchKernelGGL(deltanet_scan_kernel, dim3(ra.Hv, 128 / kScanCols), dim3(256), 0, s, ra);
     st = check_launch("deltanet_scan_kernel");
     if (st) return st;
-    hipLaunchKernelGGL(deltanet_gate_kernel, dim3((unsigned)(((size_t)ra.T * ra.Hv + 3) / 4)), dim3(256), 0, s, ra);
+    const dim3 ggrid((unsigned)(((size_t)ra.T * ra.Hv + 3) / 4));
+    const bool planes = plane_gemm_ok(hidden_size, ra.Hv * ra.D, out_dt);
+    if (planes) hipLaunchKernelGGL(deltanet_gate_kernel<true>, ggrid, dim3(256), 0, s, ra);
+    else hipLaunchKernelGGL(deltanet_gate_kernel<false>, ggrid, dim3(256), 0, s, ra);
     st = check_launch("deltanet_gate_kernel");
+    if (st) return st;
+    if (planes)
+      return launch_plane_gemm(ra.ws.planes, out_proj_weight, hidden_size, ra.T, ra.Hv * ra.D, residual, residual_dt,
+                               update, residual_out, ra.ws.part, ra.ws.part_bytes, s);
   } else {
     const int cb = ra.D < kRecCols ? ra.D : kRecCols;
     hipLaunchKernelGGL(deltanet_recurrent_kernel, dim3(ra.Hv, (ra.D + cb - 1) / cb), dim3(256), 0, s, ra);
@@ -1763,6 +1819,7 @@ static int launch_recurrent_output(const RecArgs& ra, const void* out_proj_weigh
 struct StepWs {
   StepTagWs tw;  // single-launch step: fixed-size tagged hand-off region first
   DnWs dn;
+  float* raw;    // projected qkv before the conv (where the conv is a launch of its own)
   float* mixed;
   float* z;
   float* a;
@@ -1794,6 +1851,7 @@ static size_t step_ws_layout(int T, int Hk, int Hv, int D, char* base, StepWs* w
     off = align_up(off + bytes, 256);
     return base ? reinterpret_cast<float*>(base + at) : nullptr;
   };
+  ws->raw = take((size_t)T * (2 * Hk + Hv) * D * 4);
   ws->mixed = take((size_t)T * (2 * Hk + Hv) * D * 4);
   ws->z = take((size_t)T * Hv * D * 4);
   ws->a = take((size_t)T * Hv * 4);
@@ -1963,9 +2021,7 @@ int fk_deltanet_conv(const void* mixed, int mixed_dtype, const void* conv_state,
   ca.KS = kernel_size;
   ca.out = conv_out;
   ca.next_state = next_state;
-  hipLaunchKernelGGL(deltanet_conv_kernel, dim3((channels + 255) / 256, (tokens + kConvTokens - 1) / kConvTokens),
-                     dim3(256), 0, as_stream(stream), ca);
-  return check_launch("deltanet_conv_kernel");
+  return launch_conv(ca, as_stream(stream));
 }
 
 size_t fk_deltanet_workspace_bytes(int tokens, int value_heads, int head_dim) {
@@ -2123,7 +2179,26 @@ int fk_deltanet_step(const void* hidden, const void* input_norm_weight, const vo
   pa.KS = kernel_size;
   pa.conv_out = ws.mixed;
   pa.next_state = next_conv_state;
-  st = launch_project(pa, dtypes[2], dtypes[0], s);
+  if (tokens >= kGemmMinTokens && norm_gemm_ok(pa.rows, hidden_size, dtypes[2], dtypes[1])) {
+    pa.out[0] = ws.raw;
+    st = launch_norm_gemm(hidden, dtypes[0], input_norm_weight, pa.w, pa.rows, pa.out, tokens, hidden_size, eps, 1.0f, s);
+    if (st) return st;
+    ConvArgs ca;
+    ca.mixed = ws.raw;
+    ca.mixed_dt = FK_DTYPE_F32;
+    ca.state = conv_state;
+    ca.state_dt = dtypes[3];
+    ca.w = conv_weight;
+    ca.w_dt = dtypes[4];
+    ca.T = tokens;
+    ca.C = conv_dim;
+    ca.KS = kernel_size;
+    ca.out = ws.mixed;
+    ca.next_state = next_conv_state;
+    st = launch_conv(ca, s);
+  } else {
+    st = launch_project(pa, dtypes[2], dtypes[0], s);
+  }
   if (st) return st;
 
   RecArgs ra;

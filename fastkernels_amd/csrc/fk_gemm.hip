@@ -54,24 +54,6 @@ struct GemmArgs {
 
 constexpr int kGemmBK = 64;
 
-// Eight fp32 values as three bf16 planes (packed pairs).  A value whose hi
-// term is infinite or NaN has no remainder (inf - inf would turn it to NaN).
-__device__ __forceinline__ void split3_8(const float (&v)[8], u32x4& hi, u32x4& mid, u32x4& lo) {
-  uint32_t h[4], m[4], l[4];
-#pragma unroll
-  for (int p = 0; p < 4; ++p) {
-    const float a = v[2 * p], b = v[2 * p + 1];
-    h[p] = pack_bf16x2(a, b);
-    const float ha = __uint_as_float(h[p] << 16), hb = __uint_as_float(h[p] & 0xffff0000u);
-    const float ra = fabsf(ha) < INFINITY ? a - ha : 0.f, rb = fabsf(hb) < INFINITY ? b - hb : 0.f;
-    m[p] = pack_bf16x2(ra, rb);
-    l[p] = pack_bf16x2(ra - __uint_as_float(m[p] << 16), rb - __uint_as_float(m[p] & 0xffff0000u));
-  }
-  hi = u32x4{h[0], h[1], h[2], h[3]};
-  mid = u32x4{m[0], m[1], m[2], m[3]};
-  lo = u32x4{l[0], l[1], l[2], l[3]};
-}
-
 __device__ __forceinline__ void store4(float* p, const float (&v)[4], bool vec) {
   if (vec) {
     *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
@@ -321,19 +303,32 @@ __global__ __launch_bounds__(64 * WN * WM, OCC) void token_gemm_kernel(GemmArgs 
 struct GemmReduceArgs {
   const float* part;
   int splits;
-  size_t n;  // T * R
+  size_t n;  // T * R, a multiple of 16
   float* out;
   const void* residual;
   int residual_dt;
   float* residual_out;
+  int vec;
 };
 __global__ __launch_bounds__(256) void token_gemm_reduce_kernel(GemmReduceArgs a) {
-  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
   if (i >= a.n) return;
-  float v = a.part[i];
-  for (int s = 1; s < a.splits; ++s) v += a.part[(size_t)s * a.n + i];
-  a.out[i] = v;
-  if (a.residual_out) a.residual_out[i] = load_scalar(a.residual, a.residual_dt, i) + v;
+  float4 v = *reinterpret_cast<const float4*>(a.part + i);
+  for (int s = 1; s < a.splits; ++s) {
+    const float4 p = *reinterpret_cast<const float4*>(a.part + (size_t)s * a.n + i);
+    v.x += p.x;
+    v.y += p.y;
+    v.z += p.z;
+    v.w += p.w;
+  }
+  const float o[4] = {v.x, v.y, v.z, v.w};
+  store4(a.out + i, o, a.vec);
+  if (a.residual_out) {
+    float r[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) r[q] = load_scalar(a.residual, a.residual_dt, i + q) + o[q];
+    store4(a.residual_out + i, r, a.vec);
+  }
 }
 
 // Tiles, in the order of kGemmTiles.
@@ -415,6 +410,75 @@ int launch_norm_gemm(const void* x, int x_dt, const void* nw, const void* const 
   if (x_dt == FK_DTYPE_BF16) launch_tile<0, true>(tile, a, s);
   else launch_tile<0, false>(tile, a, s);
   return check_launch("token_gemm_kernel");
+}
+
+// Tile and K splits of launch_plane_gemm.  A split is one more round of
+// partial sums through memory, but a quarter of the K steps on four times the
+// CUs where a batch has few tiles.  Estimate, us (measured at 2,048 rows, K
+// 4096, 4 to 1000 tokens; splits up to 8): the tile's time over its share of K
+// + the launch, and the reduction's launch and traffic.  us with the best
+// split and without: 32 tokens 13 / 36, 64 16 / 35, 128 20 / 35, 256 25 / 36,
+// 512 38 / 43, 1000 57.
+static void plane_tiles(int T, int R, int K, size_t part_bytes, int& tile, int& splits) {
+  constexpr float kFirst[] = {17.f, 20.5f, 25.5f, 44.f, 80.f};
+  const int cus = device_cus() > 0 ? device_cus() : 256;
+  float best = 0.f;
+  tile = -1;
+  for (int i = 0; i < (int)(sizeof(kGemmTiles) / sizeof(kGemmTiles[0])); ++i) {
+    const GemmTile& t = kGemmTiles[i];
+    const long long tiles = (long long)((R + t.bn - 1) / t.bn) * ((T + t.bm - 1) / t.bm);
+    for (int s = 1; s <= 8; s *= 2) {
+      if (s > 1 && (tiles * s > cus || K / kGemmBK < 4 * s || (size_t)s * T * R * 4 > part_bytes)) break;
+      float us = 5.f + (kFirst[i] + t.next * (float)((tiles * s + cus - 1) / cus - 1)) * (float)K / (2048.f * s);
+      if (s > 1) us += 3.f + (float)s * T * R * 8.f / 3.0e6f;
+      if (tile < 0 || us < best) {
+        best = us;
+        tile = i;
+        splits = s;
+      }
+    }
+  }
+}
+
+bool plane_gemm_ok(int R, int K, int weight_dt) {
+  return weight_dt == FK_DTYPE_BF16 && R % 16 == 0 && K >= kGemmBK && K % kGemmBK == 0;
+}
+
+int launch_plane_gemm(const uint16_t* planes, const void* w, int R, int T, int K, const void* residual,
+                      int residual_dt, float* out, float* residual_out, float* part, size_t part_bytes,
+                      hipStream_t s) {
+  GemmArgs a = {};
+  int tile;
+  plane_tiles(T, R, K, part_bytes, tile, a.splits);
+  a.w[0] = w;
+  a.rows[0] = R;
+  a.out[0] = out;
+  a.R = R;
+  a.T = T;
+  a.K = K;
+  a.planes = planes;
+  a.residual = residual;
+  a.residual_dt = residual_dt;
+  a.residual_out = residual_out;
+  a.part = a.splits > 1 ? part : nullptr;
+  const int vec = aligned16(out) && (!residual_out || aligned16(residual_out));
+  a.vec = a.part || vec;
+  a.nrb = (R + kGemmTiles[tile].bn - 1) / kGemmTiles[tile].bn;
+  a.ntb = (T + kGemmTiles[tile].bm - 1) / kGemmTiles[tile].bm;
+  launch_tile<1, false>(tile, a, s);
+  int st = check_launch("token_gemm_kernel");
+  if (st || a.splits == 1) return st;
+  GemmReduceArgs r;
+  r.part = part;
+  r.splits = a.splits;
+  r.n = (size_t)T * R;
+  r.out = out;
+  r.residual = residual;
+  r.residual_dt = residual_dt;
+  r.residual_out = residual_out;
+  r.vec = vec;
+  hipLaunchKernelGGL(token_gemm_reduce_kernel, dim3((unsigned)((r.n / 4 + 255) / 256)), dim3(256), 0, s, r);
+  return check_launch("token_gemm_reduce_kernel");
 }
 
 }  // namespace fk

@@ -40,6 +40,15 @@ bool norm_gemm_ok(const int (&rows)[4], int K, int weight_dt, int nw_dt);
 int launch_norm_gemm(const void* x, int x_dt, const void* nw, const void* const (&w)[4], const int (&rows)[4],
                      float* const (&out)[4], int T, int K, float eps, float off, hipStream_t s);
 
+// out = v . w^T (+ residual: residual_out) for a bf16 matrix of R rows and
+// values v given as bf16 planes [3][T][K] (the three terms of split3_2);
+// `part` (16-byte aligned) takes partial sums when K is split, as far as
+// part_bytes go.
+bool plane_gemm_ok(int R, int K, int weight_dt);
+int launch_plane_gemm(const uint16_t* planes, const void* w, int R, int T, int K, const void* residual,
+                      int residual_dt, float* out, float* residual_out, float* part, size_t part_bytes,
+                      hipStream_t s);
+
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 inline bool is_float_dtype(int dt) { return dt == FK_DTYPE_F32 || dt == FK_DTYPE_BF16; }

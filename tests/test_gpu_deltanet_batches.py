@@ -1,6 +1,6 @@
 """The DeltaNet operators at the edges of their token blocks: the conv's rows
 of 8, the recurrence's chunks of 16, head_dim 128 (the scan kernel) and 64
-(the general one)."""
+(the general one), and the step call at the sizes between its launches."""
 
 from __future__ import annotations
 
@@ -15,6 +15,19 @@ pytestmark = pytest.mark.gpu
 
 def _randn(gen, shape, scale=1.0, dtype=torch.float32):
     return (torch.randn(shape, generator=gen) * scale).to(dtype)
+
+
+def test_conv_in_place():
+    """The C entry with its outputs over its inputs gives what separate ones give."""
+
+    from fastkernels_amd import _lib
+
+    gen = torch.Generator().manual_seed(5)
+    mixed, state, w = (_randn(gen, s).cuda() for s in ((37, 300), (300, 4), (300, 1, 4)))
+    out, nxt = hip.hip_qwen36_batched_deltanet_conv(mixed, state, w)
+    _lib.call("fk_deltanet_conv", mixed.data_ptr(), 0, state.data_ptr(), 0, w.data_ptr(), 0, 37, 300, 4,
+              mixed.data_ptr(), state.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    assert torch.equal(mixed, out) and torch.equal(state, nxt)
 
 
 @pytest.mark.parametrize("kernel_size", [1, 4, 8])
@@ -33,12 +46,13 @@ def test_conv_blocks(tokens, kernel_size):
 
 
 @pytest.mark.parametrize("tokens,qk_heads,value_heads,head_dim", [
-    (1, 16, 32, 128), (15, 2, 4, 128), (16, 4, 4, 128), (17, 16, 32, 128), (32, 1, 2, 128), (51, 16, 32, 128),
+    (2, 16, 32, 128), (3, 16, 32, 128), (15, 2, 4, 128), (16, 4, 4, 128), (17, 16, 32, 128), (32, 1, 2, 128), (51, 16, 32, 128),
     (19, 2, 4, 64),
 ])
-def test_recurrence_chunks(tokens, qk_heads, value_heads, head_dim):
+@pytest.mark.parametrize("hidden", [256, 250])  # 250: the general output projection
+def test_recurrence_chunks(tokens, qk_heads, value_heads, head_dim, hidden):
     gen = torch.Generator().manual_seed(tokens)
-    hidden, vw = 256, value_heads * head_dim
+    vw = value_heads * head_dim
     args = dict(
         mixed_qkv=_randn(gen, (tokens, 2 * qk_heads * head_dim + vw)), z=_randn(gen, (tokens, vw)),
         a_logits=_randn(gen, (tokens, value_heads)), b_logits=_randn(gen, (tokens, value_heads)),
@@ -72,3 +86,28 @@ def test_recurrence_chunks(tokens, qk_heads, value_heads, head_dim):
     # its decay and delta forget again
     assert float((state.cpu().double() - s).norm() / s.norm()) < 2e-6
     assert float((update.cpu().double() - ref).norm() / ref.norm()) < 4e-6
+
+
+@pytest.mark.parametrize("tokens,conv_dtype", [(9, torch.bfloat16), (16, torch.bfloat16), (33, torch.float32),
+                                               (64, torch.bfloat16), (4, torch.float32)])
+def test_step_equals_staged_operators(tokens, conv_dtype):
+    """fk_deltanet_step past its single launch runs the staged kernels: the
+    same values as the operators one by one, and the same on a second call."""
+
+    from fastkernels_amd.plan import DeltaNetStepPlan
+    from fastkernels_amd.workloads import make_deltanet_weights
+
+    w = make_deltanet_weights(seed=tokens, device="cuda")
+    w["conv_state"] = w["conv_state"].to(conv_dtype)
+    x = _randn(torch.Generator().manual_seed(1), (tokens, 2048)).cuda()
+    plan = DeltaNetStepPlan(w, tokens, hidden=x)
+    for _ in range(2):
+        plan.run()
+    plan.check_device()
+    mixed, z, a, b = hip.hip_qwen36_batched_deltanet_project(
+        x, w["input_norm_weight"], w["in_proj_qkv_weight"], w["in_proj_z_weight"], w["in_proj_a_weight"], w["in_proj_b_weight"])
+    mixed, conv = hip.hip_qwen36_batched_deltanet_conv(mixed, w["conv_state"], w["conv1d_weight"])
+    update, rec = hip.hip_qwen36_batched_deltanet_recurrent_output(
+        mixed, z, a, b, w["recurrent_state"], w["out_proj_weight"], w["linear_norm_weight"], w["a_log"], w["dt_bias"])
+    assert torch.equal(plan.next_conv_state, conv) and torch.equal(plan.next_recurrent_state, rec)
+    assert torch.equal(plan.update, update) and torch.equal(plan.hidden_out, x + update)
