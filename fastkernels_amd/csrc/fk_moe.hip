@@ -62,6 +62,7 @@ struct MoeWs {
   float* sgate;         // [T] shared-expert gate sigmoid(w_g . x)
   float* act;           // [(P + T), I] SwiGLU activations
   float* y;             // [(P + T), H] per-pair down-projection outputs
+  uint16_t* planes;     // [3][T][H] fp32 hidden states as bf16 terms, read by gate/up before down writes y (same memory)
 };
 
 // Counter slots of MoeWs::tickets.
@@ -106,6 +107,7 @@ static size_t moe_ws_layout(int T, int K, int E, int I, int H, char* base, MoeWs
   ws->sgate = reinterpret_cast<float*>(take((size_t)T * 4));
   ws->act = reinterpret_cast<float*>(take((P + T) * (size_t)I * 4));
   ws->y = reinterpret_cast<float*>(take((P + T) * (size_t)H * 4));
+  ws->planes = reinterpret_cast<uint16_t*>(ws->y);
   return off;
 }
 
@@ -1054,7 +1056,7 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(ExpertArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Batched expert stage (T >= 44 tokens, bf16 weights and hidden states):
+// Batched expert stage (bf16 weights; T >= 44 bf16 or 84 fp32 tokens):
 // MFMA grouped GEMM over the routing tables.
 //
 // Weight rows are loaded row-contiguously (a wavefront's K range of a row
@@ -1067,10 +1069,12 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(ExpertArgs a) {
 // in a fixed order through LDS.
 //   gate/up: work item (slot, 16 intermediates) = 16 gate + 16 up rows, 512
 //            threads, K = H split over the 8 wavefronts; the tokens are the
-//            bf16 hidden states themselves (exact products).
+//            bf16 hidden states themselves (exact products); fp32 ones, and
+//            batches with many pairs per expert, take moe_gateup_tile_kernel.
 //   down:    work item (slot, 32 or 64 output rows), 256 threads, K = I split over
 //            the 4 wavefronts; fp32 activations enter as bf16 hi + lo
-//            columns (8 pairs per tile, ~16 mantissa bits).
+//            columns (8 pairs per tile, ~16 mantissa bits), or with fp32
+//            hidden states as three terms (16 pairs per tile, 24 bits).
 // ---------------------------------------------------------------------------
 // From this many tokens the MFMA expert kernels replace the GEMV ones (model
 // shapes: equal at 40 tokens, 1.2 us faster at 48, 3.3 at 56, 7.7 at 63).
@@ -1129,6 +1133,19 @@ __device__ __forceinline__ bool expert_slot(const ExpertArgs& a, int slot, const
   pos0 = rec.y;
   npairs = rec.z;
   return true;
+}
+
+// fp32 hidden states as three bf16 planes [3][T][H] (split3_8), for the MFMA
+// gate/up products.
+__global__ __launch_bounds__(256) void moe_split_kernel(ExpertArgs a) {
+  const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 8, n = (size_t)a.T * a.H;
+  if (i >= n) return;
+  float v[8];
+  load8_f32<false>(a.x, i, v);
+  u32x4 t[3];
+  split3_8(v, t[0], t[1], t[2]);
+#pragma unroll
+  for (int q = 0; q < 3; ++q) *reinterpret_cast<u32x4*>(a.ws.planes + q * n + i) = t[q];
 }
 
 // KS = H / 256: MFMA steps per wavefront (H = 512, 1024, 2048 -> 2, 4, 8).
@@ -1239,9 +1256,245 @@ __global__ __launch_bounds__(512) void moe_gateup_mfma_kernel(ExpertArgs a) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// Gate/up over tiles of BM pairs (fp32 hidden states, and batches whose
+// experts hold many pairs): a work item is (slot, tile of BM pairs, 64
+// intermediates) on 512 threads.  64 gate and the matching 64 up rows stream
+// through LDS in K steps of 128 (256 contiguous bytes a row), two steps ahead
+// in registers; the tile's tokens go through LDS beside them.
+// A slot's first tile of every 64 intermediates reads each weight once; the
+// tokens are read by I / 64 items instead of the I / 16 of the
+// register-resident kernel above, whose token reads at 8 KB (fp32) a token and
+// work item, not its weights, set its time (64 tokens 198 us for fp32 against
+// 142 for bf16).
+//   NP = 3: fp32 tokens as three bf16 planes (moe_split_kernel), products and
+//   sums fp32-accurate: the small terms and the large one of a K step in MFMA
+//   sums from zero, added to the accumulator by the VALU (error against 64
+//   bits as the GEMV kernel's).  NP = 1: the bf16 tokens themselves.
+// Wavefront w: intermediates 16 (w % 4) .. + 16 (gate and up rows, so SwiGLU
+// stays in registers) and half w / 4 of the columns, or of each K step when
+// the tile is one column tile (BM = 16).
+// Items: the shared expert's tiles, then the first tile of every slot, then
+// the further tiles of slots with more than BM pairs, found by a scan of the
+// counts.  The eight row blocks of an item run on one XCD.
+// ---------------------------------------------------------------------------
+constexpr int kGtRows = 64;   // intermediates per item
+constexpr int kGtK = 128;     // K step
+constexpr int kGtAhead = 2;   // weight steps in flight (two workgroups on a CU; three or four measured the same or, at one workgroup, slower)
+// Tiles of 32 pairs when the routed experts average more pairs than this,
+// else of 16 (fp32) or the register-resident kernel (bf16).  Expert stage at
+// the model's shapes, us: fp32 16 / 32 pairs 310 / 316 at 256 tokens, 323 /
+// 323 at 333, 431 / 352 at 512; bf16, registers / 32 pairs, 275 / 306, 300 /
+// 311, 390 / 336.
+constexpr int kGtWidePairs = 12;
+// fp32 hidden states take the MFMA kernels from this many tokens (expert
+// stage, GEMV / MFMA: 238 / 259 us at 64, 298 / 280 at 96, 359 / 298 at 128,
+// 562 / 310 at 256, 1035 / 352 at 512: the GEMV kernels apply the rows once
+// per pair).
+constexpr int kMfmaMinTokensF32 = 84;
+
+template <int BM, int NP>
+__global__ __launch_bounds__(512, 4) void moe_gateup_tile_kernel(ExpertArgs a, int items) {
+  constexpr int AW = kGtAhead, TM = BM / 16, CG = BM >= 32 ? 2 : 1, WT = TM / CG, KH = 2 / CG;  // column groups, their tiles, K halves
+  constexpr int XCH = BM * NP * 16, XP = (XCH + 511) / 512;                     // 16-byte token chunks per step, per thread
+  static_assert(TM % CG == 0, "columns split over two wavefront groups");
+  __shared__ u32x4 s_w[128 * 16];
+  __shared__ u32x4 s_x[XCH];
+  __shared__ int s_find[2];
+  __shared__ int s_tot[8];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int H = a.H, I = a.I, K = a.K, nrb = I / kGtRows;
+  // item (XCD-major) and row block
+  const int xcd = blockIdx.x & 7, loc = blockIdx.x >> 3;
+  const int item = (loc / nrb) * 8 + xcd, rb = loc % nrb, i0 = rb * kGtRows;
+  if (item >= items) return;
+  const int st = a.has_shared ? (a.T + BM - 1) / BM : 0;  // tiles of the shared expert
+  const char* W;
+  int pos0, npairs, tile;
+  const bool shared = item < st;
+  const size_t expert_bytes = (size_t)2 * I * H * 2;
+  if (shared) {
+    W = reinterpret_cast<const char*>(a.sgu);
+    pos0 = a.T * K;
+    npairs = a.T;
+    tile = item;
+  } else {
+    const int na = a.ws.num_active[0];
+    int slot = item - st;
+    tile = 0;
+    if (slot >= na) {
+      // further tile number `want` of the slots with more than BM pairs
+      const int want = slot - na;
+      int base = 0;
+      if (tid == 0) s_find[0] = -1;
+      for (int s0 = 0; s0 < na; s0 += 512) {
+        const int sl = s0 + tid;
+        const int c = sl < na ? a.ws.slots[sl].z : 0;
+        const int ex = c > BM ? (c + BM - 1) / BM - 1 : 0;
+        const int incl = wave_incl_scan(ex, lane);
+        if (lane == 63) s_tot[wave] = incl;
+        __syncthreads();
+        int before = base;
+        for (int w = 0; w < wave; ++w) before += s_tot[w];
+        if (want >= before + incl - ex && want < before + incl) {
+          s_find[0] = sl;
+          s_find[1] = 1 + want - (before + incl - ex);
+        }
+        for (int w = 0; w < 8; ++w) base += s_tot[w];
+        __syncthreads();
+      }
+      __syncthreads();
+      slot = s_find[0];
+      if (slot < 0) return;
+      tile = s_find[1];
+    }
+    const int4 rec = a.ws.slots[slot];
+    W = reinterpret_cast<const char*>(a.gu) + (size_t)rec.x * expert_bytes;
+    pos0 = rec.y;
+    npairs = rec.z;
+  }
+  const int p0 = tile * BM, np = min(BM, npairs - p0);
+
+  // staging addresses: weights, pass p: tile row p * 32 + tid / 16 (gate rows
+  // 0..63, up rows 64..127), 16-byte chunk tid % 16 of the step
+  uint32_t wo[4];  // byte offsets in the expert (under 2 I H 2 bytes)
+#pragma unroll
+  for (int p = 0; p < 4; ++p) {
+    const int r = p * 32 + (tid >> 4);
+    wo[p] = (uint32_t)(((r >> 6) * I + i0 + (r & 63)) * H + (tid & 15) * 8) * 2u;
+  }
+  // tokens, pass p: chunk q = p * 512 + tid = (plane, column, chunk of the step)
+  uint32_t xo[XP];  // element offsets from the planes (or x)
+  const uint32_t plane = (uint32_t)a.T * H;
+  const uint16_t* xsrc = NP == 1 ? reinterpret_cast<const uint16_t*>(a.x) : a.ws.planes;
+#pragma unroll
+  for (int p = 0; p < XP; ++p) {
+    const int q = min(p * 512 + tid, XCH - 1), col = (q >> 4) % BM, pl = (q >> 4) / BM;
+    const int pr = p0 + min(col, np - 1);  // columns past the tile's pairs repeat the last (dropped)
+    const int t = shared ? pr : a.ws.perm[pos0 + pr] / K;
+    xo[p] = pl * plane + (uint32_t)t * H + (q & 15) * 8;
+  }
+  u32x4 wr[AW][4], xr[2][XP];
+  auto load_w = [&](int k, int u) {
+    k = min(k, H - kGtK);
+#pragma unroll
+    for (int p = 0; p < 4; ++p) wr[u][p] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(W + wo[p] + k * 2));
+  };
+  auto load_x = [&](int k, int u) {
+    k = min(k, H - kGtK);
+#pragma unroll
+    for (int p = 0; p < XP; ++p) xr[u][p] = *reinterpret_cast<const u32x4*>(xsrc + xo[p] + k);
+  };
+  const int n = lane & 15, g4 = lane >> 4, rg = wave & 3, half = wave >> 2;
+  f32x4_t accg[WT], accu[WT];
+#pragma unroll
+  for (int j = 0; j < WT; ++j) accg[j] = accu[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+#pragma unroll
+  for (int u = 0; u < 2; ++u) load_x(u * kGtK, u);
+#pragma unroll
+  for (int u = 0; u < AW; ++u) load_w(u * kGtK, u);
+  for (int k0 = 0; k0 < H; k0 += AW * kGtK) {
+#pragma unroll
+    for (int u = 0; u < AW; ++u) {
+      const int k = k0 + u * kGtK;
+      if (k >= H) break;
+      if (k > 0) __syncthreads();  // the previous step's operands are read
+#pragma unroll
+      for (int p = 0; p < XP; ++p) {
+        const int q = p * 512 + tid, row = q >> 4;
+        if (XCH % 512 == 0 || q < XCH) s_x[row * 16 + ((q & 15) ^ (row & 15))] = xr[u & 1][p];
+      }
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        const int r = p * 32 + (tid >> 4);
+        s_w[r * 16 + ((tid & 15) ^ (r & 15))] = wr[u][p];
+      }
+      __syncthreads();
+      load_x(k + 2 * kGtK, u & 1);
+      load_w(k + AW * kGtK, u);
+      f32x4_t cg[WT], cu[WT], sg[WT], su[WT];  // the large term's sums, the small ones'
+#pragma unroll
+      for (int j = 0; j < WT; ++j) cg[j] = cu[j] = sg[j] = su[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ss = 0; ss < 4 / KH; ++ss) {
+        const int s = KH == 2 ? half * 2 + ss : ss, ch = s * 4 + g4;
+        const int gr = rg * 16 + n, ur = 64 + gr;
+        const bf16x8_t ag = __builtin_bit_cast(bf16x8_t, s_w[gr * 16 + (ch ^ (gr & 15))]);
+        const bf16x8_t au = __builtin_bit_cast(bf16x8_t, s_w[ur * 16 + (ch ^ (ur & 15))]);
+#pragma unroll
+        for (int q = NP - 1; q >= 0; --q)
+#pragma unroll
+          for (int j = 0; j < WT; ++j) {
+            const int row = q * BM + (CG == 2 ? half * WT + j : j) * 16 + n;
+            const bf16x8_t b = __builtin_bit_cast(bf16x8_t, s_x[row * 16 + (ch ^ (row & 15))]);
+            f32x4_t &dg = q ? sg[j] : cg[j], &du = q ? su[j] : cu[j];
+            dg = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ag, b, dg, 0, 0, 0);
+            du = __builtin_amdgcn_mfma_f32_16x16x32_bf16(au, b, du, 0, 0, 0);
+          }
+      }
+#pragma unroll
+      for (int j = 0; j < WT; ++j) {
+        accg[j] += NP == 3 ? cg[j] + sg[j] : cg[j];
+        accu[j] += NP == 3 ? cu[j] + su[j] : cu[j];
+      }
+    }
+  }
+  if constexpr (KH == 2) {  // the two K halves' sums
+    __syncthreads();
+    f32x4_t* s_acc = reinterpret_cast<f32x4_t*>(s_w);
+    if (half == 1) {
+      s_acc[rg * 128 + lane] = accg[0];
+      s_acc[rg * 128 + 64 + lane] = accu[0];
+    }
+    __syncthreads();
+    if (half == 0) {
+      accg[0] += s_acc[rg * 128 + lane];
+      accu[0] += s_acc[rg * 128 + 64 + lane];
+    }
+  }
+  if (KH == 1 || half == 0) {
+#pragma unroll
+    for (int j = 0; j < WT; ++j) {
+      const int col = (CG == 2 ? half * WT + j : j) * 16 + n;
+      if (col >= np) continue;
+      float4 v;
+      v.x = silu(accg[j][0]) * accu[j][0];
+      v.y = silu(accg[j][1]) * accu[j][1];
+      v.z = silu(accg[j][2]) * accu[j][2];
+      v.w = silu(accg[j][3]) * accu[j][3];
+      *reinterpret_cast<float4*>(a.ws.act + (size_t)(pos0 + p0 + col) * I + i0 + rg * 16 + g4 * 4) = v;
+    }
+  }
+
+  // Shared-expert gate sigmoid(w_g . x_t) of the tile's tokens.
+  if (shared && rb == 0 && a.sg) {
+    const int nch = H >> 3;
+    const bool sg_vec = a.sg_dt == FK_DTYPE_BF16 && (reinterpret_cast<uintptr_t>(a.sg) & 15u) == 0;
+    for (int c = wave; c < np; c += 8) {
+      const int t = p0 + c;
+      float d = 0.f;
+      for (int ch = lane; ch < nch; ch += kWave) {
+        float x8[8], g8[8];
+        load8_f32<NP == 1>(a.x, (size_t)t * H + (size_t)ch * 8, x8);
+        if (sg_vec) load8_f32<true>(a.sg, (size_t)ch * 8, g8);
+        else
+#pragma unroll
+          for (int q = 0; q < 8; ++q) g8[q] = load_scalar(a.sg, a.sg_dt, (size_t)ch * 8 + q);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) d = fmaf(x8[q], g8[q], d);
+      }
+      d = wave_sum(d);
+      if (lane == 0) a.ws.sgate[t] = sigmoid(d);
+    }
+  }
+}
+
 // KS = I / 128: MFMA steps per wavefront (I = 256, 512 -> 2, 4); RT: row
-// tiles of 16 output rows per work item.
-template <int KS, int RT>
+// tiles of 16 output rows per work item; NP: bf16 terms per fp32 activation:
+// 2 (bf16 hidden states), as two columns of a tile (8 pairs a tile), or 3
+// (fp32 hidden states: 24 bits), one MFMA each over a tile of 16 pairs.
+template <int KS, int RT, int NP>
 __global__ __launch_bounds__(256) void moe_down_mfma_kernel(ExpertArgs a) {
   extern __shared__ float4 s_dn_v[];
   char* s_lds = reinterpret_cast<char*>(s_dn_v);
@@ -1266,16 +1519,18 @@ __global__ __launch_bounds__(256) void moe_down_mfma_kernel(ExpertArgs a) {
   // n, lo for odd n) do not depend on the weights: the first tile's are
   // issued before the weight rows, each later tile's while the previous one
   // is computed.
+  constexpr int TP = NP == 2 ? 8 : 16;  // pairs per tile
   const int n = lane & 15, g4 = lane >> 4;
   float4 araw[KS][2];
-  auto load_act = [&](int tile) {
-    const int p = min(tile * 8 + (n >> 1), npairs - 1);
+  auto load_act_step = [&](int tile, int s) {
+    const int p = min(tile * TP + (NP == 2 ? n >> 1 : n), npairs - 1);
     const float* ar = a.ws.act + (size_t)(pos0 + p) * I + wave * kw + g4 * 8;
+    araw[s][0] = *reinterpret_cast<const float4*>(ar + s * 32);
+    araw[s][1] = *reinterpret_cast<const float4*>(ar + s * 32 + 4);
+  };
+  auto load_act = [&](int tile) {
 #pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      araw[s][0] = *reinterpret_cast<const float4*>(ar + s * 32);
-      araw[s][1] = *reinterpret_cast<const float4*>(ar + s * 32 + 4);
-    }
+    for (int s = 0; s < KS; ++s) load_act_step(tile, s);
   };
   load_act(0);
 
@@ -1294,31 +1549,60 @@ __global__ __launch_bounds__(256) void moe_down_mfma_kernel(ExpertArgs a) {
   __syncthreads();  // the partial tiles below overlap other wavefronts' areas
 
   float* s_part = reinterpret_cast<float*>(s_lds);  // [wave][row tile][16 rows][16 columns]
-  for (int tile = 0; tile * 8 < npairs; ++tile) {
-    u32x4 bv[KS];
-#pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      const float4 lo4 = araw[s][0], hi4 = araw[s][1];
-      const float v8[8] = {lo4.x, lo4.y, lo4.z, lo4.w, hi4.x, hi4.y, hi4.z, hi4.w};
-      uint32_t h[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        // hi = bf16(v), lo = bf16(v - hi), both rounded to nearest even
-        const uint32_t hi = pack_bf16x2(v8[2 * e], v8[2 * e + 1]);
-        const uint32_t lo = pack_bf16x2(v8[2 * e] - __uint_as_float(hi << 16), v8[2 * e + 1] - __uint_as_float(hi & 0xffff0000u));
-        h[e] = (n & 1) ? lo : hi;
-      }
-      bv[s] = u32x4{h[0], h[1], h[2], h[3]};
-    }
-    if ((tile + 1) * 8 < npairs) load_act(tile + 1);
+  for (int tile = 0; tile * TP < npairs; ++tile) {
     f32x4_t acc[RT];
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-      acc[rt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int rt = 0; rt < RT; ++rt) acc[rt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    auto act8 = [&](int s, float (&v)[8]) {
+      const float4 lo4 = araw[s][0], hi4 = araw[s][1];
+      v[0] = lo4.x; v[1] = lo4.y; v[2] = lo4.z; v[3] = lo4.w;
+      v[4] = hi4.x; v[5] = hi4.y; v[6] = hi4.z; v[7] = hi4.w;
+    };
+    auto mfma = [&](int rt, int s, const u32x4& b, f32x4_t& c) {
+      c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, av[rt][s]), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+    };
+    if constexpr (NP == 2) {
+      u32x4 bv[KS];
 #pragma unroll
-      for (int s = 0; s < KS; ++s)
-        acc[rt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, av[rt][s]),
-                                                          __builtin_bit_cast(bf16x8_t, bv[s]), acc[rt], 0, 0, 0);
+      for (int s = 0; s < KS; ++s) {
+        float v8[8];
+        act8(s, v8);
+        uint32_t h[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          // hi = bf16(v), lo = bf16(v - hi), both rounded to nearest even
+          const uint32_t hi = pack_bf16x2(v8[2 * e], v8[2 * e + 1]);
+          const uint32_t lo = pack_bf16x2(v8[2 * e] - __uint_as_float(hi << 16), v8[2 * e + 1] - __uint_as_float(hi & 0xffff0000u));
+          h[e] = (n & 1) ? lo : hi;
+        }
+        bv[s] = u32x4{h[0], h[1], h[2], h[3]};
+      }
+      if ((tile + 1) * TP < npairs) load_act(tile + 1);
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int s = 0; s < KS; ++s) mfma(rt, s, bv[s], acc[rt]);
+    } else {
+      // (the small terms in sums of their own, as in the gate/up kernel)
+      f32x4_t small[RT];
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) small[rt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        float v8[8];
+        act8(s, v8);
+        u32x4 hi, mid, lo;
+        split3_8(v8, hi, mid, lo);
+        load_act_step(tile + 1, s);
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+          mfma(rt, s, lo, small[rt]);
+          mfma(rt, s, mid, small[rt]);
+          mfma(rt, s, hi, acc[rt]);
+        }
+      }
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) acc[rt] += small[rt];
     }
     if (tile > 0) __syncthreads();  // the previous tile's sums are read
     float* pw = s_part + (size_t)wave * RT * 256;
@@ -1328,19 +1612,22 @@ __global__ __launch_bounds__(256) void moe_down_mfma_kernel(ExpertArgs a) {
       for (int q = 0; q < 4; ++q) pw[rt * 256 + (g4 * 4 + q) * 16 + n] = acc[rt][q];
     __syncthreads();
     // thread: output row R = tid % NR (tile R / 16, row R % 16), pairs
-    // j = tid / NR + jj * (256 / NR) (NR = 16: threads past 128 idle)
+    // j = tid / NR + jj * (256 / NR)
     {
-      constexpr int JS = 256 / NR < 8 ? 256 / NR : 8;
+      constexpr int JS = 256 / NR < TP ? 256 / NR : TP;
       const int R = tid % NR, rt = R >> 4, r = R & 15;
 #pragma unroll
-      for (int jj = 0; jj < 8 / JS; ++jj) {
+      for (int jj = 0; jj < TP / JS; ++jj) {
         const int j = tid / NR + jj * JS;
-        if (j >= 8) break;
+        if (j >= TP) break;
         float y = 0.f;
 #pragma unroll
-        for (int w = 0; w < kDnMfmaWaves; ++w)
-          y += s_part[w * RT * 256 + rt * 256 + r * 16 + 2 * j] + s_part[w * RT * 256 + rt * 256 + r * 16 + 2 * j + 1];
-        if (tile * 8 + j < npairs) a.ws.y[(size_t)(pos0 + tile * 8 + j) * H + r0 + R] = y;
+        for (int w = 0; w < kDnMfmaWaves; ++w) {
+          const float* pr = s_part + w * RT * 256 + rt * 256 + r * 16;
+          if constexpr (NP == 2) y += pr[2 * j] + pr[2 * j + 1];
+          else y += pr[j];
+        }
+        if (tile * TP + j < npairs) a.ws.y[(size_t)(pos0 + tile * TP + j) * H + r0 + R] = y;
       }
     }
   }
@@ -2634,39 +2921,67 @@ static int launch_router(const RouterArgs& ra, int router_dt, int hidden_dt, hip
   return st;
 }
 
-// Batched expert stage on MFMA: gate/up then down (see moe_gateup_mfma_kernel).
-static int launch_experts_mfma(const ExpertArgs& ea, int slots, hipStream_t stream) {
+template <int BM, int NP>
+static int launch_gateup_tile(const ExpertArgs& ea, int max_active, hipStream_t stream) {
+  // the shared expert's tiles, the slots' first tiles, and at most P / BM further ones
+  const int items = (ea.has_shared ? (ea.T + BM - 1) / BM : 0) + max_active + ea.T * ea.K / BM;
+  const dim3 grid((unsigned)((items + 7) / 8 * 8 * (ea.I / kGtRows)));
+  hipLaunchKernelGGL((moe_gateup_tile_kernel<BM, NP>), grid, dim3(512), 0, stream, ea, items);
+  return check_launch("moe_gateup_tile_kernel");
+}
+
+// Batched expert stage on MFMA: gate/up then down.
+static int launch_experts_mfma(const ExpertArgs& ea, bool bfx, int slots, hipStream_t stream) {
   static bool attr_set[64] = {false};
-  const size_t gu_shm = std::max((size_t)16 * ((size_t)ea.H * 2 + 16), (size_t)kGuMfmaWaves * 512 * sizeof(float));
-  const bool dn_small = (long long)ea.T * ea.K <= (long long)kDnMfmaSmallPairs * ea.E;
+  const int max_active = slots - (ea.has_shared ? 1 : 0);
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return fail(FK_ERR_LAUNCH, "no current HIP device");
+  int st = FK_OK;
+  const bool wide = (long long)ea.T * ea.K > (long long)kGtWidePairs * ea.E;
+  if (!bfx) {
+    const size_t n8 = (size_t)ea.T * ea.H / 8;
+    hipLaunchKernelGGL(moe_split_kernel, dim3((unsigned)((n8 + 255) / 256)), dim3(256), 0, stream, ea);
+    st = check_launch("moe_split_kernel");
+    if (st) return st;
+    st = wide ? launch_gateup_tile<32, 3>(ea, max_active, stream) : launch_gateup_tile<16, 3>(ea, max_active, stream);
+  } else if (wide) {
+    st = launch_gateup_tile<32, 1>(ea, max_active, stream);
+  } else {
+    const size_t gu_shm = std::max((size_t)16 * ((size_t)ea.H * 2 + 16), (size_t)kGuMfmaWaves * 512 * sizeof(float));
+    if (!attr_set[dev]) {
+      // (the largest need, H = 2048: 65,792 bytes)
+      const int max_gu = 16 * (2048 * 2 + 16);
+      for (const void* k : {reinterpret_cast<const void*>(moe_gateup_mfma_kernel<2>),
+                            reinterpret_cast<const void*>(moe_gateup_mfma_kernel<4>),
+                            reinterpret_cast<const void*>(moe_gateup_mfma_kernel<8>)})
+        if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, max_gu) != hipSuccess)
+          return fail(FK_ERR_LAUNCH, "cannot reserve %d bytes of LDS for the MFMA gate/up kernel", max_gu);
+      attr_set[dev] = true;
+    }
+    const dim3 gu_grid(slots * (ea.I / kGuMfmaRows)), gu_block(kGuMfmaWaves * kWave);
+    if (ea.H == 2048) hipLaunchKernelGGL(moe_gateup_mfma_kernel<8>, gu_grid, gu_block, gu_shm, stream, ea);
+    else if (ea.H == 1024) hipLaunchKernelGGL(moe_gateup_mfma_kernel<4>, gu_grid, gu_block, gu_shm, stream, ea);
+    else hipLaunchKernelGGL(moe_gateup_mfma_kernel<2>, gu_grid, gu_block, gu_shm, stream, ea);
+    st = check_launch("moe_gateup_mfma_kernel");
+  }
+  if (st) return st;
+  // (fp32: 64 rows always, so that an activation is split into its terms half
+  // as often: 104 -> 94 us at 128 tokens)
+  const bool dn_small = bfx && (long long)ea.T * ea.K <= (long long)kDnMfmaSmallPairs * ea.E;
   const int dn_rows = dn_small ? kDnMfmaRowsSmall : kDnMfmaRows;
   const size_t dn_shm = std::max((size_t)16 * kDnMfmaWaves * ((size_t)ea.I / kDnMfmaWaves * 2 + 16),
                                  (size_t)kDnMfmaWaves * dn_rows * 16 * sizeof(float));
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return fail(FK_ERR_LAUNCH, "no current HIP device");
-  if (!attr_set[dev]) {
-    // (the largest need, H = 2048: 65,792 bytes)
-    const int max_gu = 16 * (2048 * 2 + 16);
-    for (const void* k : {reinterpret_cast<const void*>(moe_gateup_mfma_kernel<2>),
-                          reinterpret_cast<const void*>(moe_gateup_mfma_kernel<4>),
-                          reinterpret_cast<const void*>(moe_gateup_mfma_kernel<8>)})
-      if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, max_gu) != hipSuccess)
-        return fail(FK_ERR_LAUNCH, "cannot reserve %d bytes of LDS for the MFMA gate/up kernel", max_gu);
-    attr_set[dev] = true;
-  }
-  const dim3 gu_grid(slots * (ea.I / kGuMfmaRows)), gu_block(kGuMfmaWaves * kWave);
-  if (ea.H == 2048) hipLaunchKernelGGL(moe_gateup_mfma_kernel<8>, gu_grid, gu_block, gu_shm, stream, ea);
-  else if (ea.H == 1024) hipLaunchKernelGGL(moe_gateup_mfma_kernel<4>, gu_grid, gu_block, gu_shm, stream, ea);
-  else hipLaunchKernelGGL(moe_gateup_mfma_kernel<2>, gu_grid, gu_block, gu_shm, stream, ea);
-  int st = check_launch("moe_gateup_mfma_kernel");
-  if (st) return st;
   const dim3 dn_grid(slots * (ea.H / dn_rows)), dn_block(kDnMfmaWaves * kWave);
-  if (dn_small) {
-    if (ea.I == 512) hipLaunchKernelGGL((moe_down_mfma_kernel<4, kDnMfmaRowsSmall / 16>), dn_grid, dn_block, dn_shm, stream, ea);
-    else hipLaunchKernelGGL((moe_down_mfma_kernel<2, kDnMfmaRowsSmall / 16>), dn_grid, dn_block, dn_shm, stream, ea);
+  constexpr int RS = kDnMfmaRowsSmall / 16, RL = kDnMfmaRows / 16;
+  if (!bfx) {
+    if (ea.I == 512) hipLaunchKernelGGL((moe_down_mfma_kernel<4, RL, 3>), dn_grid, dn_block, dn_shm, stream, ea);
+    else hipLaunchKernelGGL((moe_down_mfma_kernel<2, RL, 3>), dn_grid, dn_block, dn_shm, stream, ea);
+  } else if (dn_small) {
+    if (ea.I == 512) hipLaunchKernelGGL((moe_down_mfma_kernel<4, RS, 2>), dn_grid, dn_block, dn_shm, stream, ea);
+    else hipLaunchKernelGGL((moe_down_mfma_kernel<2, RS, 2>), dn_grid, dn_block, dn_shm, stream, ea);
   } else {
-    if (ea.I == 512) hipLaunchKernelGGL((moe_down_mfma_kernel<4, kDnMfmaRows / 16>), dn_grid, dn_block, dn_shm, stream, ea);
-    else hipLaunchKernelGGL((moe_down_mfma_kernel<2, kDnMfmaRows / 16>), dn_grid, dn_block, dn_shm, stream, ea);
+    if (ea.I == 512) hipLaunchKernelGGL((moe_down_mfma_kernel<4, RL, 2>), dn_grid, dn_block, dn_shm, stream, ea);
+    else hipLaunchKernelGGL((moe_down_mfma_kernel<2, RL, 2>), dn_grid, dn_block, dn_shm, stream, ea);
   }
   return check_launch("moe_down_mfma_kernel");
 }
@@ -2677,8 +2992,8 @@ static int launch_experts(const ExpertArgs& ea, int expert_dt, hipStream_t strea
   const int max_active = ea.T * ea.K < ea.E ? ea.T * ea.K : ea.E;
   const int slots = max_active + (ea.has_shared ? 1 : 0);
   int st = FK_OK;
-  if (ea.T >= kMfmaMinTokens && bfw && bfx && mfma_expert_shapes_ok(ea.H, ea.I)) {
-    st = launch_experts_mfma(ea, slots, stream);
+  if (ea.T >= (bfx ? kMfmaMinTokens : kMfmaMinTokensF32) && bfw && mfma_expert_shapes_ok(ea.H, ea.I)) {
+    st = launch_experts_mfma(ea, bfx, slots, stream);
     if (st) return st;
   } else {
     const int gu_grid = slots * (ea.I / kGateUpRows);

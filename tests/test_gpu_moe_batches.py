@@ -1,0 +1,80 @@
+"""Batched experts on the matrix cores with fp32 hidden states, and batches
+whose experts hold many pairs, against float64."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from fastkernels_amd.kernels import hip
+
+pytestmark = pytest.mark.gpu
+
+
+def _randn(gen, shape, scale=1.0, dtype=torch.bfloat16):
+    return (torch.randn(shape, generator=gen) * scale).to(dtype).cuda()
+
+
+def _mlp(x, gu, dn):
+    g, u = (x @ gu.double().t()).chunk(2, dim=-1)
+    return (F.silu(g) * u) @ dn.double().t()
+
+
+def _reference(x, ids, w, gu, dn, sgu=None, sdn=None, sg=None):
+    xd = x.double()
+    out = torch.zeros_like(xd)
+    for e in range(gu.shape[0]):
+        share = (w.double() * (ids == e)).sum(-1, keepdim=True)
+        t = (share != 0).nonzero()[:, 0]
+        if len(t):
+            out[t] += share[t] * _mlp(xd[t], gu[e], dn[e])
+    if sgu is not None:
+        s = _mlp(xd, sgu, sdn)
+        out += s if sg is None else torch.sigmoid(xd @ sg.double().reshape(-1, 1)) * s
+    return out
+
+
+# tiles of 16 and 32 pairs (the average pairs per expert either side of the
+# line), one pair, a tile's edge, several tiles of one expert; with and
+# without the shared expert; the shapes the kernels take
+@pytest.mark.parametrize("tokens,hidden,inter,experts,top_k,shared", [
+    (84, 2048, 512, 256, 8, True),
+    (96, 512, 256, 16, 2, True),     # 12 pairs on average: tiles of 16
+    (97, 512, 256, 16, 2, False),    # just over: tiles of 32
+    (150, 1024, 256, 4, 3, True),    # 112 pairs an expert: further tiles
+    (300, 1024, 512, 3, 2, False),
+    (512, 2048, 256, 256, 8, True),
+])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_expert_batches(tokens, hidden, inter, experts, top_k, shared, dtype):
+    gen = torch.Generator().manual_seed(tokens)
+    gu, dn = _randn(gen, (experts, 2 * inter, hidden), 0.02), _randn(gen, (experts, hidden, inter), 0.02)
+    x = _randn(gen, (tokens, hidden), 1.0, dtype)
+    ids = torch.rand((tokens, experts), generator=gen).topk(top_k, dim=-1).indices
+    ids[:17] = ids[0]  # one set of experts with more pairs than the others
+    ids, w = ids.to(torch.int32).cuda(), torch.rand((tokens, top_k), generator=gen).cuda()
+    if shared:
+        s = (_randn(gen, (2 * inter, hidden), 0.02), _randn(gen, (hidden, inter), 0.02), _randn(gen, (hidden,), 0.02))
+        out = hip.hip_qwen36_batched_routed_shared_experts_decode(x, ids, w, gu, dn, *s)
+    else:
+        s = ()
+        out = hip.hip_qwen36_batched_routed_experts_decode(x, ids, w, gu, dn)
+    ref = _reference(x, ids, w, gu, dn, *s)
+    # fp32: sums over K = H then I with about K / 100 roundings of 2^-24; bf16
+    # hidden states: the activations as two bf16 terms, 2^-18 of each rounded
+    err = float((out.double() - ref).norm() / ref.norm())
+    assert err < (1e-6 if dtype == torch.float32 else 8e-6), err
+    again = (hip.hip_qwen36_batched_routed_shared_experts_decode(x, ids, w, gu, dn, *s) if shared
+             else hip.hip_qwen36_batched_routed_experts_decode(x, ids, w, gu, dn))
+    assert torch.equal(out, again)
+
+
+def test_one_expert_takes_every_pair():
+    gen = torch.Generator().manual_seed(9)
+    gu, dn = _randn(gen, (8, 512, 512), 0.02), _randn(gen, (8, 512, 256), 0.02)
+    x = _randn(gen, (200, 512), 1.0, torch.float32)
+    ids, w = torch.full((200, 2), 5, dtype=torch.int64).cuda(), torch.rand((200, 2), generator=gen).cuda()
+    out = hip.hip_qwen36_batched_routed_experts_decode(x, ids, w, gu, dn)
+    ref = _reference(x, ids, w, gu, dn)
+    assert float((out.double() - ref).norm() / ref.norm()) < 1e-6
