@@ -7,9 +7,10 @@
 // every product with a bf16 weight is the fp32 one.  Two terms (16 bits)
 // would lose precision against the fp32 VALU products these kernels replace.
 // The MFMAs of one 64-wide K step start from zero and their sum is added to
-// the tile's fp32 accumulator by the VALU: K / 64 roundings of the full sum
-// instead of 3 K / 32 (error against 64 bits 1.33e-7 of the result, as the
-// VALU kernels'; accumulating in the MFMA throughout, 4.9e-7).
+// the tile's fp32 accumulator by the VALU, in the smaller tiles four steps at
+// a time: K / 64 roundings of the full sum or fewer instead of 3 K / 32 (error
+// against 64 bits 1.0e-7 of the result, 1.3e-7 with the largest tile; the VALU
+// kernels' 1.3e-7; accumulating in the MFMA throughout, 4.9e-7).
 //
 // Tile: BN weight rows x BM tokens per workgroup, K in steps of 64.  Both
 // operands go through LDS in 128-byte rows whose 16-byte chunks are
@@ -24,8 +25,8 @@
 // large tiles amortise (780-880 of the 1206 TFLOP/s a library bf16 GEMM
 // reaches, three MFMAs per product counted).  The DeltaNet input projections
 // (12,352 rows, K 2048) before (VALU, whole rows per wavefront) and now, us:
-// 8 tokens 41.6 / 24, 32 110 / 25, 64 201 / 30, 128 388 / 41, 256 829 / 54,
-// 512 2062 / 88, 1000 4011 / 179.
+// 8 tokens 41.6 / 26.5, 32 110 / 28, 64 201 / 32, 128 388 / 42, 256 829 / 64,
+// 512 2062 / 100, 1000 4011 / 195.
 #include "fk_common.h"
 #include "fk_host.h"
 
@@ -169,11 +170,28 @@ __global__ __launch_bounds__(64 * WN * WM, OCC) void token_gemm_kernel(GemmArgs 
 
   const int wn = wave / WM, wm = wave % WM;
   const int n = lane & 15, g4 = lane >> 4;
-  f32x4_t acc[TN][TM];
+  // Sums of four steps at a time where the registers allow (TWO), then of
+  // those: half the rounding error of one running sum of K / 64 terms.
+  constexpr bool TWO = TN * TM <= 4;
+  f32x4_t acc[TN][TM], sum[TWO ? TN : 1][TWO ? TM : 1];
 #pragma unroll
   for (int i = 0; i < TN; ++i)
 #pragma unroll
-    for (int j = 0; j < TM; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < TM; ++j) {
+      acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      if constexpr (TWO) sum[i][j] = acc[i][j];
+    }
+  auto flush = [&]() {
+    if constexpr (TWO)
+#pragma unroll
+      for (int i = 0; i < TN; ++i)
+#pragma unroll
+        for (int j = 0; j < TM; ++j) {
+          sum[i][j] += acc[i][j];
+          acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        }
+  };
+  int nstep = 0;
   auto compute = [&](int b) {
     bf16x8_t av[TN][2];
 #pragma unroll
@@ -204,6 +222,7 @@ __global__ __launch_bounds__(64 * WN * WM, OCC) void token_gemm_kernel(GemmArgs 
 #pragma unroll
       for (int i = 0; i < TN; ++i) acc[i][j] += c[i];
     }
+    if ((++nstep & 3) == 0) flush();
   };
 
   constexpr int U0 = PW > PX ? PW : PX, U = DB && U0 < 2 ? 2 : U0;
@@ -252,6 +271,13 @@ __global__ __launch_bounds__(64 * WN * WM, OCC) void token_gemm_kernel(GemmArgs 
     __syncthreads();
   }
 
+  if constexpr (TWO) {
+    flush();
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j) acc[i][j] = sum[i][j];
+  }
   float* s_rs = reinterpret_cast<float*>(&s_x[0][0]);  // (every operand is read)
   if constexpr (XM == 0) {
     // 1 / rms of the tile's tokens: the 8 threads of a row add their squares

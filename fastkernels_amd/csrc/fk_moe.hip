@@ -151,17 +151,19 @@ __device__ void build_routing_tables(const int* s_ids, int P, int E, int K, MoeW
   const int seg = (P + NWV - 1) / NWV;
   const int j0 = min(P, wave * seg), j1 = min(P, j0 + seg);
   int* wc = s_wcnt + wave * E;
+  const int ebits = E > 1 ? 32 - __builtin_clz((unsigned)(E - 1)) : 0;
   for (int c0 = j0; c0 < j1; c0 += kWave) {
     const int j = c0 + lane;
     const bool valid = j < j1;
-    const int e = valid ? s_ids[j] : -1;
-    const int n = min(kWave, j1 - c0);
-    int below = 0, total = 0;
-    for (int src = 0; src < n; ++src) {
-      const int v = __builtin_amdgcn_readlane(e, src);
-      below += (v == e) & (src < lane);
-      total += (v == e);
+    const int e = valid ? s_ids[j] : 0;
+    // the chunk's lanes with this lane's expert: one ballot per id bit (a
+    // readlane per lane took 64 rounds a chunk: 50 us for 2,664 pairs)
+    uint64_t same = __ballot(valid);
+    for (int q = 0; q < ebits; ++q) {
+      const uint64_t bit = __ballot((e >> q) & 1);
+      same &= (e >> q) & 1 ? bit : ~bit;
     }
+    const int below = __popcll(same & ((1ull << lane) - 1ull)), total = __popcll(same);
     int before = 0;
     if (valid) {
       before = wc[e];
@@ -748,15 +750,21 @@ struct AlignArgs {
   int32_t* inverse_out;
 };
 
-__global__ __launch_bounds__(256) void moe_align_kernel(AlignArgs a) {
+constexpr int kAlignWaves = 16;  // (four wavefronts and a readlane per pair: 50 us at 2,664 pairs; now 9)
+__global__ __launch_bounds__(64 * kAlignWaves) void moe_align_kernel(AlignArgs a) {
+  constexpr int NTH = 64 * kAlignWaves;
   __shared__ int s_ids[kMaxPairs];
   __shared__ int s_rank[kMaxPairs];
-  __shared__ int s_wcnt[4 * kMaxExperts];
+  __shared__ int s_wcnt[kAlignWaves * kMaxExperts];
   __shared__ int s_cnt[kMaxExperts];
   __shared__ int s_off[kMaxExperts];
   __shared__ int s_aidx[kMaxExperts];
   const int P = a.T * a.K;
-  for (int j = threadIdx.x; j < P; j += 256) {
+  for (int j = threadIdx.x; j < P; j += NTH) {
+    if (!a.ids) {  // the router's, in the workspace already
+      s_ids[j] = a.ws.ids32[j];
+      continue;
+    }
     long long v = a.ids_dt == FK_DTYPE_I64 ? reinterpret_cast<const long long*>(a.ids)[j]
                                            : (long long)reinterpret_cast<const int*>(a.ids)[j];
     int e = (int)(v < 0 ? 0 : (v >= a.E ? a.E - 1 : v));
@@ -765,10 +773,10 @@ __global__ __launch_bounds__(256) void moe_align_kernel(AlignArgs a) {
     a.ws.wts[j] = a.w ? load_scalar(a.w, a.w_dt, j) : 0.f;
   }
   __syncthreads();
-  build_routing_tables<4>(s_ids, P, a.E, a.K, a.ws, s_cnt, s_off, s_rank, s_wcnt, s_aidx);
+  build_routing_tables<kAlignWaves>(s_ids, P, a.E, a.K, a.ws, s_cnt, s_off, s_rank, s_wcnt, s_aidx);
   __syncthreads();
   // Optional copies of the tables for callers that inspect them.
-  for (int e = threadIdx.x; e < a.E; e += 256) {
+  for (int e = threadIdx.x; e < a.E; e += NTH) {
     if (a.counts_out) a.counts_out[e] = s_cnt[e];
     if (a.offsets_out) a.offsets_out[e] = s_off[e];
   }
@@ -776,11 +784,33 @@ __global__ __launch_bounds__(256) void moe_align_kernel(AlignArgs a) {
   if (a.perm_out || a.inverse_out) {
     __threadfence_block();
     __syncthreads();
-    for (int j = threadIdx.x; j < P; j += 256) {
+    for (int j = threadIdx.x; j < P; j += NTH) {
       if (a.perm_out) a.perm_out[j] = a.ws.perm[j];
       if (a.inverse_out) a.inverse_out[j] = a.ws.inverse[j];
     }
   }
+}
+
+// Top-k of every token, a wavefront each, from finished logits (the router of
+// more than 256 tokens whose logits launch_norm_gemm computed): adds the bias
+// to the logits, selects, and leaves ids and weights in the workspace for the
+// routing tables.  No waits; a workspace whose error word is set, or whose
+// wait bound is 0, still gives NaN weights and the flag, as kernels with waits.
+template <int NJE>
+__global__ __launch_bounds__(256) void moe_topk_kernel(RouterArgs a) {
+  const int lane = threadIdx.x & 63, t = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const bool bad = wait_limits(a.ws.tickets, kTicketEpoch).spin == 0u;
+  if (bad && threadIdx.x == 0)
+    __hip_atomic_fetch_or(&a.ws.tickets[kTicketError], FK_DEVICE_ERR_BARRIER, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (t >= a.T) return;
+  if (a.bias) {
+    for (int e = lane; e < a.E; e += kWave) {
+      float* p = a.logits + (size_t)t * a.E + e;
+      store_coherent(p, *p + load_scalar(a.bias, a.bias_dt, e));  // read back below by the same lane
+    }
+    publish_wait();
+  }
+  router_topk_token<NJE>(a, t, lane, bad);
 }
 
 // ---------------------------------------------------------------------------
@@ -2914,6 +2944,29 @@ static int launch_router(const RouterArgs& ra, int router_dt, int hidden_dt, hip
   }
   const bool wide = ra.H > 2048, many = ra.E > 256;
   int st = FK_OK;
+  // Batches past the tagged router: logits as MFMA tiles (fp32-accurate),
+  // selections and tables as launches of their own (512 tokens of the model's
+  // shape: 179 -> 43 us against the grid-barrier kernel below, whose VALU
+  // logits take ~0.3 us a token and whose last workgroup builds the tables).
+  const int rows[4] = {ra.E, 0, 0, 0};
+  if (norm_gemm_ok(rows, ra.H, router_dt, ra.nw_dt)) {
+    const void* const w[4] = {ra.W, nullptr, nullptr, nullptr};
+    float* const out[4] = {ra.logits, nullptr, nullptr, nullptr};
+    st = launch_norm_gemm(ra.x, hidden_dt, ra.nw, w, rows, out, ra.T, ra.H, ra.eps, ra.off, stream);
+    if (st) return st;
+    const dim3 grid((unsigned)((ra.T + 3) / 4));
+    if (many) hipLaunchKernelGGL(moe_topk_kernel<16>, grid, dim3(256), 0, stream, ra);
+    else hipLaunchKernelGGL(moe_topk_kernel<4>, grid, dim3(256), 0, stream, ra);
+    st = check_launch("moe_topk_kernel");
+    if (st) return st;
+    AlignArgs aa = {};
+    aa.T = ra.T;
+    aa.K = ra.K;
+    aa.E = ra.E;
+    aa.ws = ra.ws;
+    hipLaunchKernelGGL(moe_align_kernel, dim3(1), dim3(64 * kAlignWaves), 0, stream, aa);
+    return check_launch("moe_align_kernel");
+  }
   FK_DISPATCH_BOOL(bfw, BW, FK_DISPATCH_BOOL(bfx, BX, {
     if (wide) st = many ? launch_router_t<BW, BX, 8, 16>(ra, stream) : launch_router_t<BW, BX, 8, 4>(ra, stream);
     else st = many ? launch_router_t<BW, BX, 4, 16>(ra, stream) : launch_router_t<BW, BX, 4, 4>(ra, stream);
@@ -3203,7 +3256,7 @@ int fk_moe_align(const void* topk_ids, int ids_dtype, const void* topk_weights, 
   aa.offsets_out = offsets_out;
   aa.perm_out = perm_out;
   aa.inverse_out = inverse_out;
-  hipLaunchKernelGGL(moe_align_kernel, dim3(1), dim3(256), 0, as_stream(stream), aa);
+  hipLaunchKernelGGL(moe_align_kernel, dim3(1), dim3(64 * kAlignWaves), 0, as_stream(stream), aa);
   return check_launch("moe_align_kernel");
 }
 

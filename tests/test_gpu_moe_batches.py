@@ -78,3 +78,41 @@ def test_one_expert_takes_every_pair():
     out = hip.hip_qwen36_batched_routed_experts_decode(x, ids, w, gu, dn)
     ref = _reference(x, ids, w, gu, dn)
     assert float((out.double() - ref).norm() / ref.norm()) < 1e-6
+
+
+@pytest.mark.parametrize("pairs,experts", [(1, 1), (63, 3), (64, 256), (65, 2), (1023, 7), (1030, 1024), (4096, 256), (4096, 1)])
+def test_routing_tables(pairs, experts):
+    from oracle import qwen36 as oracle
+
+    gen = torch.Generator().manual_seed(pairs)
+    top_k = 8 if pairs % 8 == 0 else 1  # (a token may name an expert twice here)
+    ids = torch.randint(0, experts, (pairs // top_k, top_k), generator=gen)
+    got = hip.hip_qwen36_moe_align(ids.cuda(), experts)
+    for g, r in zip(got, oracle.moe_align(ids, experts)):
+        assert torch.equal(g.cpu(), torch.from_numpy(r))
+
+
+# past the tagged router's 256 tokens: logits as tiles, then the selection
+@pytest.mark.parametrize("tokens,hidden,experts,top_k,bias,dtype", [
+    (257, 2048, 256, 8, False, torch.float32),
+    (300, 512, 48, 3, True, torch.bfloat16),
+    (512, 1024, 1024, 8, True, torch.float32),
+    (20, 64, 272, 8, False, torch.float32),
+])
+def test_router_batches(tokens, hidden, experts, top_k, bias, dtype):
+    from oracle import qwen36 as oracle
+
+    gen = torch.Generator().manual_seed(tokens)
+    x, norm = _randn(gen, (tokens, hidden), 1.0, dtype), _randn(gen, (hidden,), 0.1)
+    w = _randn(gen, (experts, hidden), 0.05)
+    b = _randn(gen, (experts,), 0.5, torch.float32) if bias else None
+    logits, ids, weights = hip.hip_qwen36_batched_moe_router_decode(x, norm, w, top_k=top_k, router_bias=b)
+    ref, _, _ = oracle.router(x.cpu(), norm.cpu(), w.cpu(), top_k, router_bias=None if b is None else b.cpu(), dtype=torch.float64)
+    # 2^-24 of sum |w| |x| per rounding of the K / 64 partial sums
+    bound = (hidden / 64 + 20) * 2.0 ** -24 * hidden ** 0.5 * 0.05 * hidden ** 0.5
+    assert float((logits.cpu().double() - ref).abs().max()) < bound
+    own = torch.softmax(logits.cpu().double(), -1)
+    val, own_ids = oracle.topk_lowest_id(torch.softmax(logits.cpu(), -1), top_k)
+    assert torch.equal(ids.cpu(), own_ids)
+    pick = own.gather(1, own_ids)
+    assert torch.allclose(weights.cpu().double(), pick / pick.sum(-1, keepdim=True), rtol=1e-5, atol=0)
