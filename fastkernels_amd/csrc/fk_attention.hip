@@ -14,7 +14,9 @@
 //   update = (o * sigmoid(gate)) Wo^T;  hidden_out = x + update
 //
 // Kernels: T <= 4 at the shapes attn_step_chunks accepts (the model's) run
-// as one launch, attn_step_kernel (below); other steps as four launches:
+// as one launch, attn_step_kernel (below); 8 rows or more at the shapes
+// attn_prompt_ok accepts as matrix products (fk_attention_prompt.hip); other
+// steps as four launches:
 //   attn_proj_kernel  RMSNorm folded into a GEMV over [Wq | Wk | Wv] (9216
 //                     rows at the model shape); H > 2048 takes the shared
 //                     normalized projection kernel of fk_deltanet.hip
@@ -41,6 +43,10 @@ namespace fk {
 constexpr int kAttnMaxHeadDim = 256;
 constexpr int kAttnMaxTokens = 32;  // new keys of the step are kept in LDS (T * hd floats)
 constexpr int kAttnOutRows = 4;  // Wo rows per out-projection workgroup (1 per wavefront)
+// From this many rows launch_attn_prompt's kernels replace the four launches
+// below (58 against 68 us at 5 rows behind 1,000 positions, 65 / 61 at 8
+// behind 100, 126 / 73 at 16, 195 / 71 at 32).
+constexpr int kPromptMinTokens = 8;
 
 struct AttnArgs {
   const float* qg;      // [T, heads * 2 * hd] projected query/gate pairs
@@ -1358,6 +1364,7 @@ struct AttnWs {
   float* v;
   float* gated;
   float* part;
+  char* prompt;  // launch_attn_prompt's workspace (calls past the single launch)
 };
 
 static size_t attn_ws_layout(int T, int heads, int kvh, int hd, char* base, AttnWs* ws) {
@@ -1382,6 +1389,10 @@ static size_t attn_ws_layout(int T, int heads, int kvh, int hd, char* base, Attn
   ws->v = floats((size_t)T * kvh * hd);
   ws->gated = floats((size_t)T * heads * hd);
   ws->part = floats((size_t)T * heads * kAttnMaxChunks * (hd + 2));
+  // (hd 256 and G a divisor of 64 are what launch_attn_prompt takes; smaller
+  // shapes never need it)
+  const bool prompt = T >= kPromptMinTokens && hd == kAttnMaxHeadDim && kvh > 0 && heads % kvh == 0 && heads / kvh <= 8;
+  ws->prompt = take(prompt ? attn_prompt_ws_bytes(T, heads, kvh) : 0);
   return off;
 }
 
@@ -1543,6 +1554,10 @@ int fk_attention_decode(const void* hidden, int hidden_dtype, const void* norm_w
     return fail(FK_ERR_INVALID, "projection pointers must be non-NULL");
   if (!aligned16(hidden) || !aligned16(norm_weight) || !aligned16(q_proj) || !aligned16(k_proj) || !aligned16(v_proj))
     return fail(FK_ERR_ALIGNMENT, "hidden, norm_weight and projection weights must be 16-byte aligned");
+  const AttnPromptCall call = {hidden, hidden_dtype, norm_weight, q_proj, k_proj, v_proj, o_proj, q_norm_weight, k_norm_weight,
+                               qk_norm_dtype, key_cache, value_cache, cache_dtype, max_positions, start_position,
+                               start_position_device, tokens, hidden_size, heads, kv_heads, rd - rd % 2, rope_interleaved,
+                               rope_theta, eps, qk_eps, update, hidden_out, ws.tw.tickets + kWorkspaceErrorWord};
   if (tokens <= kAsMaxTokens) {
     const bool bx = hidden_dtype == FK_DTYPE_BF16, cb = cache_dtype == FK_DTYPE_BF16;
     const int G = attn_step_grid_for(bx, cb);
@@ -1585,6 +1600,8 @@ int fk_attention_decode(const void* hidden, int hidden_dtype, const void* norm_w
       return check_launch("attn_step_kernel");
     }
   }
+  if (tokens >= kPromptMinTokens && attn_prompt_ok(tokens, hidden_size, heads, kv_heads, head_dim, weight_dtype, norm_dtype))
+    return launch_attn_prompt(call, ws.prompt, s);
   st = fk_attention_project(hidden, hidden_dtype, norm_weight, norm_dtype, q_proj, k_proj, v_proj, weight_dtype,
                             tokens, hidden_size, 2 * heads * head_dim, kv_heads * head_dim, eps, 1.0f, ws.qg, ws.k,
                             ws.v, stream);
@@ -1664,6 +1681,49 @@ int fk_attention_decode(const void* hidden, int hidden_dtype, const void* norm_w
   if (weight_dtype == FK_DTYPE_BF16) hipLaunchKernelGGL(attn_out_kernel<true>, ogrid, dim3(256), 0, s, o);
   else hipLaunchKernelGGL(attn_out_kernel<false>, ogrid, dim3(256), 0, s, o);
   return check_launch("attn_out_kernel");
+}
+
+// Workspace header words before launch_attn_prompt's region (the error word
+// of the workspace convention lies in it).
+static constexpr size_t kPromptHeader = 256;
+
+size_t fk_attention_prompt_workspace_bytes(int tokens, int hidden_size, int heads, int kv_heads, int head_dim,
+                                           int weight_dtype, int norm_dtype) {
+  if (!attn_prompt_ok(tokens, hidden_size, heads, kv_heads, head_dim, weight_dtype, norm_dtype)) return 0;
+  return kPromptHeader + attn_prompt_ws_bytes(tokens, heads, kv_heads);
+}
+
+int fk_attention_prompt(const void* hidden, int hidden_dtype, const void* norm_weight, int norm_dtype,
+                        const void* q_proj, const void* k_proj, const void* v_proj, const void* o_proj,
+                        int weight_dtype, const void* q_norm_weight, const void* k_norm_weight, int qk_norm_dtype,
+                        void* key_cache, void* value_cache, int cache_dtype, int max_positions, int start_position,
+                        int tokens, int hidden_size, int heads, int kv_heads, int head_dim, int rope_dim,
+                        float rope_theta, int rope_interleaved, float eps, float qk_eps, float* update,
+                        float* hidden_out, void* workspace, size_t workspace_bytes, void* stream) {
+  if (tokens < 1) return fail(FK_ERR_INVALID, "tokens must be positive");
+  if (rope_dim < 0) return fail(FK_ERR_INVALID, "rope_dim must be >= 0");
+  if (max_positions < 1 || start_position < 0 || (long long)start_position + tokens > max_positions)
+    return fail(FK_ERR_INVALID, "positions [%d, %lld) exceed the cache length %d", start_position,
+                (long long)start_position + tokens, max_positions);
+  if (!is_float_dtype(hidden_dtype) || !is_float_dtype(cache_dtype) || !is_float_dtype(qk_norm_dtype))
+    return fail(FK_ERR_DTYPE, "hidden, caches and q/k norms must be f32 or bf16");
+  const size_t need = fk_attention_prompt_workspace_bytes(tokens, hidden_size, heads, kv_heads, head_dim, weight_dtype, norm_dtype);
+  if (!need) return fail(FK_ERR_UNSUPPORTED, "not a shape fk_attention_prompt takes (use fk_attention_decode)");
+  if (!rope_interleaved && rope_dim % 2) return fail(FK_ERR_INVALID, "half-split RoPE needs an even rope_dim");
+  if (!hidden || !norm_weight || !q_proj || !k_proj || !v_proj || !o_proj || !q_norm_weight || !k_norm_weight || !key_cache ||
+      !value_cache || !update)
+    return fail(FK_ERR_INVALID, "attention pointers must be non-NULL");
+  for (const void* q : {hidden, norm_weight, q_proj, k_proj, v_proj, o_proj, (const void*)key_cache, (const void*)value_cache})
+    if (!aligned16(q)) return fail(FK_ERR_ALIGNMENT, "hidden, the weights and the caches must be 16-byte aligned");
+  if (!workspace || workspace_bytes < need)
+    return fail(FK_ERR_WORKSPACE, "attention workspace needs %zu bytes (got %zu)", need, workspace ? workspace_bytes : 0);
+  if (!aligned16(workspace)) return fail(FK_ERR_ALIGNMENT, "workspace must be 16-byte aligned");
+  const int rd = rope_dim < head_dim ? rope_dim : head_dim;
+  const AttnPromptCall call = {hidden, hidden_dtype, norm_weight, q_proj, k_proj, v_proj, o_proj, q_norm_weight, k_norm_weight,
+                               qk_norm_dtype, key_cache, value_cache, cache_dtype, max_positions, start_position, nullptr,
+                               tokens, hidden_size, heads, kv_heads, rd - rd % 2, rope_interleaved, rope_theta, eps, qk_eps,
+                               update, hidden_out, reinterpret_cast<uint32_t*>(workspace) + kWorkspaceErrorWord};
+  return launch_attn_prompt(call, reinterpret_cast<char*>(workspace) + kPromptHeader, as_stream(stream));
 }
 
 }  // extern "C"

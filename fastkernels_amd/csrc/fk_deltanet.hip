@@ -47,13 +47,6 @@ struct DnWs {
   size_t part_bytes;
 };
 
-// Partial sums of the output projection for 2,048 output rows: up to 8 splits
-// of K, fewer as the tokens fill the chip by themselves (launch_plane_gemm).
-static size_t dn_part_bytes(int T) {
-  const size_t splits = T >= 1024 ? 1 : T <= 128 ? 8 : (size_t)(1024 / T);
-  return splits > 1 ? splits * (size_t)T * 2048 * 4 : 0;
-}
-
 static size_t dn_ws_layout(int T, int Hv, int D, char* base, DnWs* ws) {
   size_t off = 0;
   auto take = [&](size_t bytes) {
@@ -65,7 +58,7 @@ static size_t dn_ws_layout(int T, int Hv, int D, char* base, DnWs* ws) {
   ws->core = reinterpret_cast<float*>(take((size_t)T * Hv * D * 4));
   ws->planes = reinterpret_cast<uint16_t*>(take((size_t)T * Hv * D * 6));
   ws->normed = reinterpret_cast<float*>(ws->planes);
-  ws->part_bytes = dn_part_bytes(T);
+  ws->part_bytes = token_part_bytes(T);
   ws->part = reinterpret_cast<float*>(take(ws->part_bytes));
   return off;
 }

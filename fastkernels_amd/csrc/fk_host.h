@@ -49,6 +49,35 @@ int launch_plane_gemm(const uint16_t* planes, const void* w, int R, int T, int K
                       int residual_dt, float* out, float* residual_out, float* part, size_t part_bytes,
                       hipStream_t s);
 
+// Bytes for launch_plane_gemm's partial sums of 2,048 output rows: up to 8
+// splits of K, fewer as the tokens fill the chip by themselves.
+inline size_t token_part_bytes(int T) {
+  const size_t splits = T >= 1024 ? 1 : T <= 128 ? 8 : (size_t)(1024 / T);
+  return splits > 1 ? splits * (size_t)T * 2048 * 4 : 0;
+}
+
+// Gated attention over T rows of one sequence as a prompt
+// (fk_attention_prompt.hip), at the shapes attn_prompt_ok takes; `err` is the
+// word that a device-held position past the cache is flagged in.
+struct AttnPromptCall {
+  const void* x;
+  int x_dt;
+  const void* nw;  // bf16
+  const void *wq, *wk, *wv, *wo;  // bf16
+  const void *qn_w, *kn_w;
+  int qk_dt;
+  void *kc, *vc;
+  int cache_dt, max_pos, start;
+  const int* start_dev;
+  int T, hidden, heads, kvh, rope_dim, interleaved;
+  float theta, eps, qk_eps;
+  float *update, *hidden_out;
+  uint32_t* err;
+};
+bool attn_prompt_ok(int T, int hidden, int heads, int kvh, int hd, int weight_dt, int norm_dt);
+size_t attn_prompt_ws_bytes(int T, int heads, int kvh);
+int launch_attn_prompt(const AttnPromptCall& p, void* workspace, hipStream_t s);
+
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 inline bool is_float_dtype(int dt) { return dt == FK_DTYPE_F32 || dt == FK_DTYPE_BF16; }

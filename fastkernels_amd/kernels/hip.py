@@ -1015,13 +1015,32 @@ def _attention(hidden, key_cache, value_cache, norm_weight, q_proj_weight, k_pro
     dev = x.device
     update = torch.empty((tokens, hidden_size), device=dev, dtype=torch.float32)
     out = torch.empty_like(update) if residual else None
-    # The C ABI decodes at most _MAX_ATTN_ROWS rows per call (their new keys
-    # sit in LDS); longer batches go through in consecutive calls: each call
+    lib = _lib.load()
+    if tokens > _MAX_ATTN_ROWS:
+        # a prompt: one call for any number of rows, at the shapes it takes
+        nbytes = lib.fk_attention_prompt_workspace_bytes(
+            tokens, hidden_size, attention_heads, kv_heads, head_dim, _fcode(wq, "projection weights"),
+            _fcode(nw, "norm_weight"))
+        if nbytes:
+            ws = _workspace("attention_prompt", dev, nbytes)
+            _lib.call(
+                "fk_attention_prompt",
+                x.data_ptr(), _fcode(x, "hidden"), nw.data_ptr(), _fcode(nw, "norm_weight"),
+                wq.data_ptr(), wk.data_ptr(), wv.data_ptr(), wo.data_ptr(), _fcode(wq, "projection weights"),
+                qn.data_ptr(), kn.data_ptr(), _fcode(qn, "q_norm_weight"),
+                kc.data_ptr(), vc.data_ptr(), _fcode(kc, "key_cache"), kc.shape[0], int(start_position),
+                tokens, hidden_size, attention_heads, kv_heads, head_dim, int(rope_dim), float(rope_theta),
+                1 if rope_interleaved else 0, float(eps), float(qk_norm_eps),
+                update.data_ptr(), _ptr(out), ws.data_ptr(), ws.numel(), _stream(dev),
+            )
+            return update, out, kc, vc
+    # fk_attention_decode takes at most _MAX_ATTN_ROWS rows per call (their new
+    # keys sit in LDS on its general path); longer batches go through in consecutive calls: each call
     # writes its rows' keys and values into the cache before the next one
     # reads them, which is the causal order one call keeps.
     # No rows: no call (the caches are returned as given, or copied).
     step = _MAX_ATTN_ROWS
-    nbytes = _lib.load().fk_attention_workspace_bytes(min(max(tokens, 1), step), attention_heads, kv_heads, head_dim)
+    nbytes = lib.fk_attention_workspace_bytes(min(max(tokens, 1), step), attention_heads, kv_heads, head_dim)
     ws = _workspace("attention", dev, nbytes)
     for s in range(0, tokens, step):
         e = min(tokens, s + step)

@@ -263,7 +263,8 @@ size_t fk_attention_workspace_bytes(int tokens, int heads, int kv_heads, int hea
  * 8 (a multiple of 4 above 4) and heads * head_dim a multiple of 512 (the
  * model's shapes) this is one launch whose workgroups hand values to each
  * other (the workspace then also carries the error word of
- * fk_workspace_status); other calls run four launches.
+ * fk_workspace_status); more tokens at the shapes fk_attention_prompt takes run
+ * its kernels, other calls four launches.
  * Replaces triton_qwen36_batched_attention_decode (qwen36_attention.py:448-577)
  * and the residual add of triton_qwen36_batched_attention_moe_layer_decode
  * (qwen36_layer.py:109-201). */
@@ -275,6 +276,30 @@ int fk_attention_decode(const void* hidden, int hidden_dtype,
                         void* key_cache, void* value_cache, int cache_dtype,
                         int max_positions, int start_position,
                         const int32_t* start_position_device, int tokens, int hidden_size,
+                        int heads, int kv_heads, int head_dim, int rope_dim, float rope_theta,
+                        int rope_interleaved, float eps, float qk_eps,
+                        float* update, float* hidden_out,
+                        void* workspace, size_t workspace_bytes, void* stream);
+
+/* Bytes of workspace for fk_attention_prompt, or 0 for a shape it does not
+ * take (head_dim 256, heads / kv_heads a power of two up to 8, bf16 weights
+ * and norm weight, hidden_size a multiple of 64). */
+size_t fk_attention_prompt_workspace_bytes(int tokens, int hidden_size, int heads, int kv_heads, int head_dim,
+                                           int weight_dtype, int norm_dtype);
+
+/* fk_attention_decode for any number of rows in one call (a prompt, or a
+ * chunk of one behind `start_position` cached positions), as matrix products:
+ * the same arguments without the device-held position.  Every row's own keys
+ * and values enter unrounded, and are written to the caches.  No wait between
+ * workgroups.  No counterpart in the reference beyond its batched attention
+ * decode (qwen36_attention.py:448-577). */
+int fk_attention_prompt(const void* hidden, int hidden_dtype,
+                        const void* norm_weight, int norm_dtype,
+                        const void* q_proj, const void* k_proj, const void* v_proj,
+                        const void* o_proj, int weight_dtype,
+                        const void* q_norm_weight, const void* k_norm_weight, int qk_norm_dtype,
+                        void* key_cache, void* value_cache, int cache_dtype,
+                        int max_positions, int start_position, int tokens, int hidden_size,
                         int heads, int kv_heads, int head_dim, int rope_dim, float rope_theta,
                         int rope_interleaved, float eps, float qk_eps,
                         float* update, float* hidden_out,

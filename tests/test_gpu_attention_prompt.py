@@ -1,0 +1,133 @@
+"""Attention over many rows of one sequence in one call, against the oracle's
+maths in float64 and against calls of a few rows."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from fastkernels_amd import _lib
+from fastkernels_amd.kernels import hip
+from fastkernels_amd.plan import AttentionStepPlan
+
+pytestmark = pytest.mark.gpu
+
+
+def _randn(gen, shape, scale=1.0, dtype=torch.bfloat16):
+    return (torch.randn(shape, generator=gen) * scale).to(dtype).cuda()
+
+
+def _inputs(seed, tokens, hidden, heads, kvh, positions, x_dtype, cache_dtype):
+    gen = torch.Generator().manual_seed(seed)
+    w = dict(
+        norm_weight=_randn(gen, (hidden,), 0.1), q_proj_weight=_randn(gen, (2 * heads * 256, hidden), 0.02),
+        k_proj_weight=_randn(gen, (kvh * 256, hidden), 0.02), v_proj_weight=_randn(gen, (kvh * 256, hidden), 0.02),
+        out_proj_weight=_randn(gen, (hidden, heads * 256), 0.02), q_norm_weight=_randn(gen, (256,), 0.1),
+        k_norm_weight=_randn(gen, (256,), 0.1))
+    x = _randn(gen, (tokens, hidden), 1.0, x_dtype)
+    kc, vc = (_randn(gen, (positions, kvh, 256), 1.0, cache_dtype) for _ in range(2))
+    return x, kc, vc, w
+
+
+def _reference(x, kc, vc, w, start, heads, kvh, rope_dim, theta, interleaved):
+    d = {k: v.double() for k, v in w.items()}
+    norm = lambda v, g: v * torch.rsqrt((v * v).mean(-1, keepdim=True) + 1e-6) * (1.0 + g)  # noqa: E731
+    tokens, xd = x.shape[0], x.double()
+    xn = norm(xd, d["norm_weight"])
+    q, gate = (xn @ d["q_proj_weight"].t()).reshape(tokens, heads, 512).split(256, dim=-1)
+    k, v = ((xn @ d[n].t()).reshape(tokens, kvh, 256) for n in ("k_proj_weight", "v_proj_weight"))
+    pos = torch.arange(start, start + tokens, device=x.device)
+
+    def rope(y):
+        freq = theta ** (-torch.arange(0, rope_dim, 2, dtype=torch.float64, device=y.device) / rope_dim)
+        cs, sn = ((pos.double()[:, None] * freq).cos()[:, None], (pos.double()[:, None] * freq).sin()[:, None])
+        out, h = y.clone(), rope_dim // 2
+        ia, ib = (slice(0, rope_dim, 2), slice(1, rope_dim, 2)) if interleaved else (slice(0, h), slice(h, rope_dim))
+        out[..., ia], out[..., ib] = y[..., ia] * cs - y[..., ib] * sn, y[..., ia] * sn + y[..., ib] * cs
+        return out
+
+    q, k = rope(norm(q, d["q_norm_weight"])), rope(norm(k, d["k_norm_weight"]))
+    keys, values = kc.double(), vc.double()
+    keys[start:start + tokens], values[start:start + tokens] = k, v
+    n = start + tokens
+    dead = torch.arange(n, device=x.device)[None] > pos[:, None]
+    o = torch.stack([torch.softmax((q[:, h] @ keys[:n, h * kvh // heads].t() / 16.0).masked_fill(dead, -torch.inf), -1)
+                     @ values[:n, h * kvh // heads] for h in range(heads)], 1)
+    return (o * torch.sigmoid(gate)).reshape(tokens, -1) @ d["out_proj_weight"].t(), k, v
+
+
+# rows: a row block's edges (64 / G tokens), one call of a few rows (the
+# decode entry), many; contexts: none, inside a tile, several chunks
+@pytest.mark.parametrize("tokens,start,hidden,heads,kvh,x_dtype,cache_dtype,interleaved", [
+    (5, 0, 2048, 16, 2, torch.float32, torch.float32, True),
+    (8, 37, 512, 8, 1, torch.bfloat16, torch.float32, True),
+    (32, 300, 2048, 16, 2, torch.float32, torch.bfloat16, True),
+    (33, 0, 2048, 16, 2, torch.float32, torch.float32, False),
+    (65, 15, 1024, 4, 4, torch.bfloat16, torch.bfloat16, True),
+    (200, 1000, 2048, 16, 2, torch.float32, torch.float32, True),
+    (131, 777, 512, 8, 4, torch.float32, torch.bfloat16, False),
+])
+def test_prompt_rows(tokens, start, hidden, heads, kvh, x_dtype, cache_dtype, interleaved):
+    x, kc, vc, w = _inputs(tokens, tokens, hidden, heads, kvh, start + tokens + 3, x_dtype, cache_dtype)
+    kw = dict(start_position=start, attention_heads=heads, kv_heads=kvh, rope_dim=64, rope_theta=1e4, rope_interleaved=interleaved)
+    update, k2, v2 = hip.hip_qwen36_batched_attention_decode(x, kc, vc, *w.values(), **kw)
+    ref, k, v = _reference(x, kc, vc, w, start, heads, kvh, 64, 1e4, interleaved)
+    # 32-bit products and sums; the RoPE angles are 32-bit (2^-24 of the position)
+    tol = 2e-6 + (start + tokens) * 2.0 ** -24 * 0.5
+    assert float((update.double() - ref).norm() / ref.norm()) < tol
+    rows = slice(start, start + tokens)
+    rtol = (4e-3 if cache_dtype == torch.bfloat16 else 1e-6) + (start + tokens) * 2.0 ** -23
+    for got, want, old in ((k2, k, kc), (v2, v, vc)):
+        assert torch.allclose(got[rows].double(), want, rtol=rtol, atol=rtol)
+        assert torch.equal(got[:start], old[:start]) and torch.equal(got[start + tokens:], old[start + tokens:])
+    again = hip.hip_qwen36_batched_attention_decode(x, kc, vc, *w.values(), **kw)
+    assert torch.equal(update, again[0])
+
+
+def test_rows_see_no_later_row():
+    """A later row that is not finite, or just other, changes no earlier row."""
+
+    x, kc, vc, w = _inputs(3, 40, 512, 8, 1, 90, torch.float32, torch.float32)
+    kw = dict(start_position=50, attention_heads=8, kv_heads=1, rope_dim=64)
+    good = hip.hip_qwen36_batched_attention_decode(x, kc, vc, *w.values(), **kw)[0]
+    bad = x.clone()
+    bad[21], bad[30:] = float("nan"), 3.0
+    got = hip.hip_qwen36_batched_attention_decode(bad, kc, vc, *w.values(), **kw)[0]
+    assert torch.equal(got[:21], good[:21])
+    assert bool(got[21:].isnan().all())
+
+
+@pytest.mark.parametrize("tokens", [8, 32])
+def test_device_position_advances_and_is_checked(tokens):
+    x, kc, vc, w = _inputs(7, tokens, 2048, 16, 2, 4 * tokens, torch.bfloat16, torch.float32)
+    names = {"norm_weight": "input_norm_weight", "out_proj_weight": "o_proj_weight"}
+    plan = AttentionStepPlan({names.get(k, k): v for k, v in w.items()}, tokens, max_positions=4 * tokens - 1, hidden=x)
+    plan.run()
+    stream = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        plan.run(stream)
+    graph.replay()
+    graph.replay()
+    assert int(plan.position) == 3 * tokens
+    plan.check_device()
+    spec = plan.spec
+    k, v = torch.zeros_like(plan.key_cache), torch.zeros_like(plan.value_cache)
+    for step in range(3):
+        update, k, v = hip.hip_qwen36_batched_attention_decode(
+            x, k, v, *w.values(), start_position=step * tokens, rope_theta=spec.rope_theta)
+    assert torch.equal(plan.key_cache, k) and torch.allclose(plan.update, update, rtol=1e-4, atol=1e-5)
+    graph.replay()  # past the cache: NaN, caches untouched, position left, flagged
+    torch.cuda.synchronize()
+    assert bool(plan.update.isnan().all()) and int(plan.position) == 3 * tokens and torch.equal(plan.key_cache, k)
+    with pytest.raises(_lib.FastKernelsError) as info:
+        plan.check_device()
+    assert info.value.status == _lib.FK_ERR_DEVICE
+
+
+def test_entry_refuses_what_it_does_not_take():
+    lib = _lib.load()
+    assert lib.fk_attention_prompt_workspace_bytes(40, 2048, 16, 2, 128, 1, 1) == 0
+    assert lib.fk_attention_prompt_workspace_bytes(40, 2048, 16, 2, 256, 0, 1) == 0
+    assert lib.fk_attention_prompt_workspace_bytes(0, 2048, 16, 2, 256, 1, 1) == 0
+    assert lib.fk_attention_prompt_workspace_bytes(40, 2048, 16, 2, 256, 1, 1) > 0
