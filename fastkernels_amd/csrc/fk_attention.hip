@@ -653,7 +653,9 @@ __global__ __launch_bounds__(256) void attn_out_kernel(AttnOutArgs a) {
 //       once per position; wavefronts 0-3 normalise and rotate the queries,
 //       4-7 the step's own keys, recomputed from k (its own values come from
 //       v: no dependence on another workgroup's cache write); 8 wavefronts
-//       each keep an online softmax over their positions, merged through
+//       each keep an online softmax over their positions (short chunks by
+//       tiles of kAsTile on the VALU, long ones of four heads of 256 on the
+//       matrix cores), merged through
 //       LDS.  The chunk's (max, sum, weighted values) per head leave tagged,
 //       and the chunk holding position start + t writes that token's cache
 //       rows of kv head j.
@@ -680,6 +682,13 @@ constexpr int kAsMDims = 64;       // head dims per merge unit
 constexpr int kAsKcu = 512;        // Wo columns per C1 unit
 constexpr int kAsRb = 128;         // Wo rows per C1 unit (16 per wavefront)
 constexpr int kAsTile = 24;        // cached positions per LDS tile of an attention unit
+// Chunks of more positions than this (a third tile for the loop over tiles,
+// which waits for its cached rows once per tile past the first) take the
+// pipelined MFMA softmax.  Both sides, us per step, bf16 cache and hidden
+// 2048: chunks of 40 positions 24.75 by tiles, 24.75 by MFMA; 44 (4 tokens)
+// 33.1 and 33.8; 52 26.4 and 25.0; 57 (4 tokens) 34.5 and 33.2; 188 35.8 and
+// 30.5; 750 (4 tokens) 86.1 and 59.3.
+constexpr int kAsLongMin = 2 * kAsTile;
 constexpr int kAsMaxH = 2048;
 constexpr int kAsMaxG = 8;         // query heads per kv head
 constexpr int kAsGu = 4;           // query heads per attention unit
@@ -995,6 +1004,20 @@ __global__ __launch_bounds__(kAsThreads) void attn_step_kernel(AttnStepArgs a) {
     float* s_acc = s_vn + kAsMaxTokens * hd;       // [waves][Gu][hd] wavefront states after the last tile
     // own positions of the chunk: o_lo .. p_hi - 1, tokens u_lo ..
     const int o_lo = max(p_lo, start), n_own = p_hi > o_lo ? p_hi - o_lo : 0, u_lo = o_lo - start;
+    const bool long_chunk = p_hi - p_lo > kAsLongMin && hd == kAttnMaxHeadDim && Gu == kAsGu;  // (uniform)
+    const int pc_hi = min(p_hi, o_lo);  // end of the chunk's cached positions
+    Row4<CBF> lk[2][2][4], lv[2][8];
+    auto issue_long = [&](Row4<CBF>(&kr)[2][4], Row4<CBF>(&vr)[8], int pt) __attribute__((always_inline)) {
+      const int pw = pt + wave * 8;
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const size_t row = ((size_t)min(pw + q * 4 + (lane & 3), pc_hi - 1) * kvh + aj) * hd + (lane >> 2) * 4;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) kr[q][u] = load_row4<CBF>(a.kc, row + u * 64);
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) vr[i] = load_row4<CBF>(a.vc, ((size_t)min(pw + i, pc_hi - 1) * kvh + aj) * hd + lane * 4);
+    };
     // token at's queries of heads hb .. (word e = g * hd + d), the own
     // tokens' k and v (word e = s * hd + d), polled directly (their first
     // round of loads in flight while the RoPE angles are computed)
@@ -1014,7 +1037,10 @@ __global__ __launch_bounds__(kAsThreads) void attn_step_kernel(AttnStepArgs a) {
     // inputs and staged after the norms and RoPE.  (Issued behind the phase
     // A weight rows instead, it was waited for with them: the attention
     // units then ended phase A last, 1.4 us later at ctx 1024.)
-    issue_tile(p_lo);
+    if (long_chunk)
+      issue_long(lk[0], lv[0], p_lo);
+    else
+      issue_tile(p_lo);
     // RoPE angles, once per position: slot 0 the queries' (apos), slot
     // 1 + s own key s's (o_lo + s); entry i of a slot is pair i's (cos, sin)
     {
@@ -1074,57 +1100,165 @@ __global__ __launch_bounds__(kAsThreads) void attn_step_kernel(AttnStepArgs a) {
       m[g] = -INFINITY;
       l[g] = 0.f;
     }
-    // tiles of kAsTile positions (the first issued with the inputs):
-    // wavefront w takes positions pt + w, + 8, .. from its registers; per
-    // head one softmax step over its positions of the tile.  The step's own
-    // positions read the recomputed keys and the values from v.
-    for (int pt = p_lo; pt < p_hi; pt += kAsTile) {
-      if (pt != p_lo) issue_tile(pt);
-      FK_MARK(12);
-      const int pend = min(pt + kAsTile, p_hi);
-      float sr[PPW];  // lanes 16g ..: head g's score at position pt + w + 8 bb
+    float lm = -INFINITY, ll = 0.f;  // (long chunks: the lane's head's state)
+    f32x4_t lo[4];
+    if (long_chunk) {
+      // Long chunks on v_mfma_f32_4x4x1 (16 blocks of 4 x 4, fp32 in and
+      // out): the four query heads are the four columns, so no lane is idle,
+      // where a 16 x 16 tile would waste three quarters of its columns.
+      // Lane l = 4 b + c:
+      //   scores of four keys: block b sums dims 64 u + 4 b + e (u, e < 4),
+      //     A = key c's (16 bytes a load), B = head c's query; the blocks are
+      //     then added, and register r of every lane with l % 4 = h holds key
+      //     r's score for head h
+      //   values: A = V[key][4 l + u], B = the key's probability for head c;
+      //     lo[u][r] = dim 4 (4 b + r) + u of head c
+      // Wavefront w takes positions pt + 8 w .. + 8 of a tile of 64, the next
+      // tile's rows in flight (two register sets).  The loop over tiles below
+      // is bound by VALU issue (a dot product per head and position, one
+      // wavefront pair per SIMD) and by a memory round trip per 24 positions:
+      // 12,000 positions took 35.8 us a step with it (bf16 cache), 30.5 here;
+      // 4 tokens 86.1 -> 59.3.
+      const int blk = lane >> 2, hc = lane & 3;
+      float4 qv[4];
 #pragma unroll
-      for (int bb = 0; bb < PPW; ++bb) {
-        const int p = min(pt + wave + kAsWaves * bb, pend - 1);  // (positions past the tile: scored -inf below)
-        const float4 k4 = p >= o_lo ? *reinterpret_cast<const float4*>(s_kf + (p - o_lo) * hd + dl) : ckr[bb].f4();  // (uniform)
-        float d[kAsGu];
+      for (int u = 0; u < 4; ++u) qv[u] = *reinterpret_cast<const float4*>(s_qf + hc * hd + u * 64 + blk * 4);
 #pragma unroll
-        for (int g = 0; g < kAsGu; ++g) d[g] = q4[g].x * k4.x + q4[g].y * k4.y + q4[g].z * k4.z + q4[g].w * k4.w;
-        sr[bb] = rows4_sum(d);
+      for (int u = 0; u < 4; ++u) lo[u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      // four keys: their scores for the lane's head (all blocks added)
+      auto scores4 = [&](const float4 (&k4)[4], f32x4_t& out) __attribute__((always_inline)) {
+        f32x4_t s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          f32x4_t& su = u & 1 ? s1 : s0;
+          su = __builtin_amdgcn_mfma_f32_4x4x1f32(k4[u].x, qv[u].x, su, 0, 0, 0);
+          su = __builtin_amdgcn_mfma_f32_4x4x1f32(k4[u].y, qv[u].y, su, 0, 0, 0);
+          su = __builtin_amdgcn_mfma_f32_4x4x1f32(k4[u].z, qv[u].z, su, 0, 0, 0);
+          su = __builtin_amdgcn_mfma_f32_4x4x1f32(k4[u].w, qv[u].w, su, 0, 0, 0);
+        }
+        out = s0 + s1;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          float v = out[r];
+          v += __uint_as_float(dpp_u32<0x124>(__float_as_uint(v)));  // row_ror:4
+          v += __uint_as_float(dpp_u32<kDppRowRor8>(__float_as_uint(v)));
+          v += __uint_as_float(xor16_u32(__float_as_uint(v)));
+          out[r] = v + __uint_as_float(xor32_u32(__float_as_uint(v)));
+        }
+      };
+      // softmax step over N keys (scores -inf where masked) and their values
+      auto fold = [&](const f32x4_t* sc, const float4* v4, auto n_tag) __attribute__((always_inline)) {
+        constexpr int N = decltype(n_tag)::value;
+        float mx = lm;
+#pragma unroll
+        for (int i = 0; i < N; ++i) mx = fmaxf(mx, sc[i >> 2][i & 3]);
+        const float f = lm == -INFINITY ? 0.f : __expf(lm - mx);
+        ll *= f;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) lo[u] *= f;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+          const float s = sc[i >> 2][i & 3], p = s == -INFINITY ? 0.f : __expf(s - mx);
+          ll += p;
+          lo[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(v4[i].x, p, lo[0], 0, 0, 0);
+          lo[1] = __builtin_amdgcn_mfma_f32_4x4x1f32(v4[i].y, p, lo[1], 0, 0, 0);
+          lo[2] = __builtin_amdgcn_mfma_f32_4x4x1f32(v4[i].z, p, lo[2], 0, 0, 0);
+          lo[3] = __builtin_amdgcn_mfma_f32_4x4x1f32(v4[i].w, p, lo[3], 0, 0, 0);
+        }
+        lm = mx;
+      };
+      auto tile = [&](const Row4<CBF>(&kr)[2][4], const Row4<CBF>(&vr)[8], int pt) __attribute__((always_inline)) {
+        const int pw = pt + wave * 8;
+        if (pw >= pc_hi) return;  // (uniform: none of the tile's positions are this wavefront's)
+        f32x4_t sc[2];
+        float4 v4[8];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          float4 k4[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) k4[u] = kr[q][u].f4();
+          scores4(k4, sc[q]);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) sc[q][r] = pw + q * 4 + r < pc_hi ? sc[q][r] : -INFINITY;
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v4[i] = vr[i].f4();
+        fold(sc, v4, std::integral_constant<int, 8>{});
+      };
+      if (wave == kAsWaves - 1 && n_own > 0) {  // the step's own positions (at most four)
+        float4 k4[4], v4[4];
+        f32x4_t sc[1];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          k4[u] = *reinterpret_cast<const float4*>(s_kf + min(hc, n_own - 1) * hd + u * 64 + blk * 4);
+        scores4(k4, sc[0]);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          sc[0][r] = r < n_own ? sc[0][r] : -INFINITY;
+          v4[r] = *reinterpret_cast<const float4*>(s_vn + min(r, n_own - 1) * hd + lane * 4);
+        }
+        fold(sc, v4, std::integral_constant<int, 4>{});
       }
-#pragma unroll
-      for (int g = 0; g < kAsGu; ++g) {
-        if (g >= Gu) break;
-        float sc[PPW];
-        float mx = m[g];
+      for (int pt = p_lo; pt < pc_hi; pt += 128) {
+        issue_long(lk[1], lv[1], pt + 64);
+        tile(lk[0], lv[0], pt);
+        if (pt + 64 >= pc_hi) break;
+        issue_long(lk[0], lv[0], pt + 128);
+        tile(lk[1], lv[1], pt + 64);
+      }
+    } else {
+      // tiles of kAsTile positions (the first issued with the inputs):
+      // wavefront w takes positions pt + w, + 8, .. from its registers; per
+      // head one softmax step over its positions of the tile.  The step's own
+      // positions read the recomputed keys and the values from v.
+      for (int pt = p_lo; pt < p_hi; pt += kAsTile) {
+        if (pt != p_lo) issue_tile(pt);
+        FK_MARK(12);
+        const int pend = min(pt + kAsTile, p_hi);
+        float sr[PPW];  // lanes 16g ..: head g's score at position pt + w + 8 bb
 #pragma unroll
         for (int bb = 0; bb < PPW; ++bb) {
-          sc[bb] = pt + wave + kAsWaves * bb < pend
-                       ? __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(sr[bb]), 16 * g))
-                       : -INFINITY;
-          mx = fmaxf(mx, sc[bb]);
-        }
-        if (mx == -INFINITY) continue;  // (uniform: no position of this wavefront in the tile)
-        const float f = __expf(m[g] - mx);
-        float es = 0.f;
-        float4 av = make_float4(0.f, 0.f, 0.f, 0.f);
+          const int p = min(pt + wave + kAsWaves * bb, pend - 1);  // (positions past the tile: scored -inf below)
+          const float4 k4 = p >= o_lo ? *reinterpret_cast<const float4*>(s_kf + (p - o_lo) * hd + dl) : ckr[bb].f4();  // (uniform)
+          float d[kAsGu];
 #pragma unroll
-        for (int bb = 0; bb < PPW; ++bb) {
-          const int p = min(pt + wave + kAsWaves * bb, pend - 1);
-          const float e = __expf(sc[bb] - mx);
-          const float4 v4 = p >= o_lo ? *reinterpret_cast<const float4*>(s_vn + (p - o_lo) * hd + dl) : cvr[bb].f4();  // (uniform)
-          es += e;
-          av.x = fmaf(e, v4.x, av.x);
-          av.y = fmaf(e, v4.y, av.y);
-          av.z = fmaf(e, v4.z, av.z);
-          av.w = fmaf(e, v4.w, av.w);
+          for (int g = 0; g < kAsGu; ++g) d[g] = q4[g].x * k4.x + q4[g].y * k4.y + q4[g].z * k4.z + q4[g].w * k4.w;
+          sr[bb] = rows4_sum(d);
         }
-        l[g] = l[g] * f + es;
-        acc[g].x = acc[g].x * f + av.x;
-        acc[g].y = acc[g].y * f + av.y;
-        acc[g].z = acc[g].z * f + av.z;
-        acc[g].w = acc[g].w * f + av.w;
-        m[g] = mx;
+#pragma unroll
+        for (int g = 0; g < kAsGu; ++g) {
+          if (g >= Gu) break;
+          float sc[PPW];
+          float mx = m[g];
+#pragma unroll
+          for (int bb = 0; bb < PPW; ++bb) {
+            sc[bb] = pt + wave + kAsWaves * bb < pend
+                         ? __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(sr[bb]), 16 * g))
+                         : -INFINITY;
+            mx = fmaxf(mx, sc[bb]);
+          }
+          if (mx == -INFINITY) continue;  // (uniform: no position of this wavefront in the tile)
+          const float f = __expf(m[g] - mx);
+          float es = 0.f;
+          float4 av = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+          for (int bb = 0; bb < PPW; ++bb) {
+            const int p = min(pt + wave + kAsWaves * bb, pend - 1);
+            const float e = __expf(sc[bb] - mx);
+            const float4 v4 = p >= o_lo ? *reinterpret_cast<const float4*>(s_vn + (p - o_lo) * hd + dl) : cvr[bb].f4();  // (uniform)
+            es += e;
+            av.x = fmaf(e, v4.x, av.x);
+            av.y = fmaf(e, v4.y, av.y);
+            av.z = fmaf(e, v4.z, av.z);
+            av.w = fmaf(e, v4.w, av.w);
+          }
+          l[g] = l[g] * f + es;
+          acc[g].x = acc[g].x * f + av.x;
+          acc[g].y = acc[g].y * f + av.y;
+          acc[g].z = acc[g].z * f + av.z;
+          acc[g].w = acc[g].w * f + av.w;
+          m[g] = mx;
+        }
       }
     }
     lds_barrier();  // the softmax states reuse the row tile
@@ -1132,14 +1266,25 @@ __global__ __launch_bounds__(kAsThreads) void attn_step_kernel(AttnStepArgs a) {
     // the wavefronts' states merged per (head, dim): per-wavefront factors
     // exp(m_w - M) once, then the chunk partial (max, sum, weighted values)
     // leaves tagged
+    if (long_chunk) {
+      if (lane < 4) {
+        s_m[wave][lane] = lm;
+        s_l[wave][lane] = ll;
+      }
 #pragma unroll
-    for (int g = 0; g < kAsGu; ++g) {
-      if (g < Gu) {
-        if (lane == 0) {
-          s_m[wave][g] = m[g];
-          s_l[wave][g] = l[g];
+      for (int r = 0; r < 4; ++r)
+        *reinterpret_cast<float4*>(s_acc + ((size_t)wave * Gu + (lane & 3)) * hd + ((lane >> 2) * 4 + r) * 4) =
+            make_float4(lo[0][r], lo[1][r], lo[2][r], lo[3][r]);
+    } else {
+#pragma unroll
+      for (int g = 0; g < kAsGu; ++g) {
+        if (g < Gu) {
+          if (lane == 0) {
+            s_m[wave][g] = m[g];
+            s_l[wave][g] = l[g];
+          }
+          if (lin) *reinterpret_cast<float4*>(s_acc + ((size_t)wave * Gu + g) * hd + d0) = acc[g];
         }
-        if (lin) *reinterpret_cast<float4*>(s_acc + ((size_t)wave * Gu + g) * hd + d0) = acc[g];
       }
     }
     lds_barrier();

@@ -84,6 +84,28 @@ def test_prompt_rows(tokens, start, hidden, heads, kvh, x_dtype, cache_dtype, in
     assert torch.equal(update, again[0])
 
 
+# step calls with long chunks of positions per workgroup (64, 32, 21 and 16
+# chunks for 1 to 4 tokens): the last chunk length of the loop over tiles (48)
+# and the first past it, tiles of 64 positions with every kind of remainder,
+# a last chunk of own positions, of few positions and an empty one, groups of
+# 2 and 4 query heads
+@pytest.mark.parametrize("tokens,start,hidden,heads,kvh,cache_dtype", [
+    (1, 3071, 2048, 16, 2, torch.float32),
+    (1, 3072, 2048, 16, 2, torch.float32),
+    (1, 3527, 2048, 16, 2, torch.bfloat16),
+    (1, 4095, 2048, 16, 2, torch.bfloat16),
+    (1, 4096, 2048, 16, 2, torch.float32),
+    (2, 2100, 2048, 16, 2, torch.float32),
+    (3, 1640, 2048, 16, 2, torch.bfloat16),
+    (4, 1037, 2048, 16, 2, torch.float32),
+    (4, 12000, 2048, 16, 2, torch.float32),
+    (1, 12000, 2048, 16, 2, torch.bfloat16),
+    (1, 9000, 2048, 16, 8, torch.float32),
+])
+def test_step_of_long_chunks(tokens, start, hidden, heads, kvh, cache_dtype):
+    test_prompt_rows(tokens, start, hidden, heads, kvh, torch.float32, cache_dtype, True)
+
+
 def test_rows_see_no_later_row():
     """A later row that is not finite, or just other, changes no earlier row."""
 
