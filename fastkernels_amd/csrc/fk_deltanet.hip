@@ -19,7 +19,9 @@
 //                             window in registers.
 //   deltanet_scan_kernel      head_dim 128: 16 lanes hold a column of a head's
 //                             state, no barrier per token; its raw outputs go
-//                             through deltanet_gate_kernel (gated RMSNorm).
+//                             through deltanet_gate_kernel (gated RMSNorm);
+//   deltanet_chunk_kernel,    the same by chunks of 16 tokens on the matrix
+//   deltanet_chunk_scan_kernel  cores, from kChunkMinTokens.
 //   deltanet_recurrent_kernel other head sizes and bf16 inputs: grid (Hv,
 //                             ceil(D/32)); a workgroup owns a
 //                             D x 32 fp32 state tile in registers (16 rows per
@@ -95,6 +97,10 @@ constexpr int kGemmMinTokens = 4;
 // takes 28 us from 3 to 32 tokens where the two kernels before took 24.5 us at
 // 1 and 2 (host-bound there), 30 at 3, 57 at 8 and 192 at 32.
 constexpr int kScanMinTokens = 3;
+// From this many tokens the recurrence goes by chunks of 16 (one more launch):
+// the operator takes 39.0 us at 64 tokens that way and 38.6 by tokens, 47.4 and
+// 49.6 at 96, 51.8 and 56.0 at 128, 72 and 86 at 256, 113 and 148 at 512.
+constexpr int kChunkMinTokens = 96;
 
 template <bool BFW, bool BFX, int NJ>
 __global__ __launch_bounds__(256) void deltanet_project_kernel(ProjArgs a) {
@@ -641,6 +647,308 @@ __global__ __launch_bounds__(256) void deltanet_scan_kernel(RecArgs a) {
 #pragma unroll
   for (int i = 0; i < 8; ++i)
     store_scalar(a.next_state, a.dt[4], sbase + (size_t)((i >> 2) * 64 + sub * 4 + (i & 3)) * D, S[i]);
+}
+
+// The scan of longer batches by chunks of 16 tokens on v_mfma_f32_16x16x4
+// (fp32 in and out).  With S the state before a chunk, d_t the tokens' decays,
+// P(t, j) = d_(j+1) .. d_t and D_t = d_0 .. d_t:
+//   delta_t = beta_t (v_t - D_t k_t.S) - sum_(j < t) beta_t P(t, j) (k_t.k_j) delta_j
+//   o_t     = D_t q_t.S + sum_(j <= t) P(t, j) (q_t.k_j) delta_j
+//   S'      = D_15 S + sum_j P(15, j) k_j delta_j^T
+// so only k.S, q.S and the last line wait for the chunk before.  The inverse
+// of the unit triangle I + [beta P (k.k)] turns the first line into a product;
+// its entries are at most 1 in size (products of contractions between
+// normalised keys), and the P are products of the decays themselves, as the
+// scan by tokens forms them.  deltanet_chunk_kernel computes what does not
+// depend on the state for all chunks at once.
+struct ChunkTable {      // per (chunk, value head); rows are tokens
+  float inv[16][16];     // the triangle's inverse without its diagonal of ones (16 sums with it as a
+                         // term would each round at the size of the result)
+  float qk[16][16];      // P(t, j) (q_t.k_j) for j <= t
+  float beta[16], dec[16], tail[16];  // beta_t (0 past the last token), D_t, P(15, j)
+};
+
+// Bytes of the normalised q and k rows and the tables of T tokens; they lie in
+// the planes' region, which the gate kernel fills later (enough from 2 value
+// heads per qk head; other shapes keep the scan by tokens).
+static size_t dn_chunk_bytes(int T, int Hk, int Hv) {
+  return (size_t)T * Hk * 2 * 128 * 4 + (size_t)((T + 15) / 16) * Hv * sizeof(ChunkTable);
+}
+
+__device__ __forceinline__ float* chunk_rows(const RecArgs& a) { return reinterpret_cast<float*>(a.ws.planes); }
+__device__ __forceinline__ ChunkTable* chunk_tables(const RecArgs& a) {
+  return reinterpret_cast<ChunkTable*>(chunk_rows(a) + (size_t)a.T * a.Hk * 256);
+}
+
+// Workgroup (chunk, qk head): normalised q and k rows, k.k and q.k of the
+// chunk (a wavefront each for half the dims), then a wavefront per value head
+// of the group.  It is bound by the chain of the triangle's inverse (~120
+// FMAs of a wavefront).
+__global__ __launch_bounds__(256) void deltanet_chunk_kernel(RecArgs a) {
+  constexpr int D = 128, LD = D + 4;
+  __shared__ __align__(16) float s_qk[2][16][LD];  // q, k
+  __shared__ float s_dot[4][16][17];               // k.k and q.k of dims 0 .. 63, then of 64 .. 127
+  __shared__ __align__(16) float s_a[4][16][16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tc = blockIdx.x * 16, qk_head = blockIdx.y, rep = a.Hv / a.Hk;
+  const size_t mixed_w = (size_t)2 * a.Hk * D + (size_t)a.Hv * D;
+  {
+    const int tl = tid >> 4, sub = tid & 15, t = min(tc + tl, a.T - 1);
+    const float* row = reinterpret_cast<const float*>(a.mixed) + (size_t)t * mixed_w;
+    float x[2][8];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const float4 v = *reinterpret_cast<const float4*>(row + (size_t)(i * a.Hk + qk_head) * D + sub * 8 + j * 4);
+        x[i][j * 4] = v.x;
+        x[i][j * 4 + 1] = v.y;
+        x[i][j * 4 + 2] = v.z;
+        x[i][j * 4 + 3] = v.w;
+      }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      float ss = 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) ss = fmaf(x[i][j], x[i][j], ss);
+      // (scales and beta through 64 bits: their errors are common to a whole
+      // row, and make up for the two more roundings of a delta here)
+      const float sc = (float)(1. / sqrt(((double)row16_sum(ss) + a.eps) * (i == 0 ? (double)D : 1.)));
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const float4 v = make_float4(x[i][j * 4] * sc, x[i][j * 4 + 1] * sc, x[i][j * 4 + 2] * sc, x[i][j * 4 + 3] * sc);
+        *reinterpret_cast<float4*>(&s_qk[i][tl][sub * 8 + j * 4]) = v;
+        if (tc + tl < a.T)
+          *reinterpret_cast<float4*>(chunk_rows(a) + (((size_t)t * a.Hk + qk_head) * 2 + i) * D + sub * 8 + j * 4) = v;
+      }
+    }
+  }
+  __syncthreads();
+  const int r16 = lane & 15, g = lane >> 4;
+  {
+    const int kind = wave & 1;  // 0: k.k, 1: q.k
+    f32x4_t acc[8];  // chains of two, summed in pairs
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int d = (wave >> 1) * 64 + i * 16 + g * 4;
+      const f32x4_t ta = *reinterpret_cast<const f32x4_t*>(&s_qk[kind ^ 1][r16][d]);
+      const f32x4_t tb = *reinterpret_cast<const f32x4_t*>(&s_qk[1][r16][d]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        acc[i * 2 + (e >> 1)] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+            ta[e], tb[e], e & 1 ? acc[i * 2 + (e >> 1)] : f32x4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+    }
+    acc[0] = ((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7]));
+#pragma unroll
+    for (int r = 0; r < 4; ++r) s_dot[wave][g * 4 + r][r16] = acc[0][r];
+  }
+  __syncthreads();
+  for (int v0 = 0; v0 < rep; v0 += 4) {  // (the barrier below is uniform)
+    const int h = qk_head * rep + v0 + wave;
+    const bool mine = v0 + wave < rep;
+    float dec = 1.f, beta = 0.f;  // of token tc + r16
+    if (mine && tc + r16 < a.T) {
+      const size_t ab = (size_t)(tc + r16) * a.Hv + h;
+      dec = expf(-expf(load_scalar(a.a_log, a.dt[7], h)) *
+                 softplus_stable(load_scalar(a.a_in, a.dt[2], ab) + load_scalar(a.dt_bias, a.dt[8], h)));
+      beta = (float)(1. / (1. + exp(-(double)load_scalar(a.b_in, a.dt[3], ab))));
+    }
+    ChunkTable* tab = chunk_tables(a) + (size_t)blockIdx.x * a.Hv + (mine ? h : 0);
+    if (mine) {
+      // lane (column j = r16, rows 4 g .. + 4): P(t, j) and D_t, in 64 bits:
+      // where the scan by tokens rounds every value of the state after each
+      // decay, independently, an error here would be common to a token's
+      // whole row (in 32 bits the state's error grew by 5%)
+      double p = 1., dd = 1., pk[4] = {0., 0., 0., 0.}, dk = 1.;
+#pragma unroll
+      for (int t = 0; t < 16; ++t) {
+        const double dt = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(dec), t));
+        p = t > r16 ? p * dt : p;
+        dd *= dt;
+        pk[t & 3] = t >> 2 == g && t >= r16 ? p : pk[t & 3];
+        dk = t == r16 ? dd : dk;
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int t = g * 4 + r;
+        const double bt = __shfl(beta, t);
+        const double kk = (double)s_dot[0][t][r16] + s_dot[2][t][r16], qk = (double)s_dot[1][t][r16] + s_dot[3][t][r16];
+        s_a[wave][t][r16] = t > r16 ? (float)(bt * pk[r] * kk) : 0.f;
+        tab->qk[t][r16] = t >= r16 ? (float)(pk[r] * qk) : 0.f;
+      }
+      if (g == 0) {
+        tab->beta[r16] = beta;
+        tab->dec[r16] = (float)dk;
+        tab->tail[r16] = (float)p;
+      }
+    }
+    __syncthreads();
+    if (mine) {
+      float x[16];  // column r16 of the inverse
+#pragma unroll
+      for (int t = 0; t < 16; ++t) {
+        f32x4_t s4 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int q = 0; q < (t + 3) / 4; ++q) {
+          const f32x4_t ar = *reinterpret_cast<const f32x4_t*>(&s_a[wave][t][q * 4]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (q * 4 + e < t) s4[e] = fmaf(ar[e], x[q * 4 + e], s4[e]);
+        }
+        // (rows above the diagonal stay 0 whatever the later rows hold)
+        x[t] = t < r16 ? 0.f : t == r16 ? 1.f : -((s4[0] + s4[1]) + (s4[2] + s4[3]));
+        if (g == t >> 2) tab->inv[t][r16] = t == r16 ? 0.f : x[t];
+      }
+    }
+  }
+}
+
+// Workgroup (value head, 16 columns of its state), wavefront w the state's
+// rows 32 w .. + 32 as two 16 x 16 tiles in the accumulators' layout (lane
+// l: column l % 16, register r: row 4 (l / 16) + r), which is the B operand's
+// layout too if step r of a product takes rows 4 g + r: the state, the deltas
+// and their right-hand sides go from product to product without a move.  A
+// chunk costs a wavefront 16 MFMAs for k.S and q.S, the sum over the four
+// wavefronts through LDS (one barrier), 4 for the deltas and 8 for the state;
+// the next two chunks' operands are in flight meanwhile.  What bounds it: the
+// chain of a chunk (1.6 us; with one chunk in flight 1.7).  512 tokens: 51 us
+// and 10 of deltanet_chunk_kernel, by tokens 100; the operator 148 -> 113 us.
+// Errors against 64 bits at 16 to 512 tokens: state 7.2e-8 to 8.2e-8 (by
+// tokens 7.4e-8 to 9.0e-8), update 1.8e-7 (1.7e-7; two launches with barriers
+// per token, which both replace, 2.4e-7).
+__global__ __launch_bounds__(256) void deltanet_chunk_scan_kernel(RecArgs a) {
+  constexpr int D = 128;
+  __shared__ f32x4_t s_part[2][4][2][64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int r16 = lane & 15, g = lane >> 4;
+  const int h = blockIdx.x, col = blockIdx.y * 16 + r16;
+  const int qk_head = h / (a.Hv / a.Hk);
+  const size_t mixed_w = (size_t)2 * a.Hk * D + (size_t)a.Hv * D;
+  const float* vcol = reinterpret_cast<const float*>(a.mixed) + (size_t)2 * a.Hk * D + (size_t)h * D + col;
+  const float* qrow = chunk_rows(a) + (size_t)qk_head * 2 * D + wave * 32;
+  const size_t rstep = (size_t)a.Hk * 2 * D;
+  const size_t sbase = (size_t)h * D * D + (size_t)(wave * 32 + g * 4) * D + col;
+
+  f32x4_t S[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) S[i][r] = load_scalar(a.state, a.dt[4], sbase + (size_t)(i * 16 + r) * D);
+
+  struct Operands {
+    f32x4_t q[2], k[2];  // rows' dims 16 i + 4 g .. + 4 of token r16
+    f32x4_t kt[2];       // dim 16 i + r16 of tokens 4 g .. + 4
+    f32x4_t v;           // column of tokens 4 g .. + 4
+    f32x4_t inv, qk;     // columns 4 g .. + 4 of row r16
+    f32x4_t beta, dec, tail;
+    float last;
+  };
+  auto fetch = [&](Operands& o, int c) __attribute__((always_inline)) {
+    const int tc = min(c * 16, (a.T - 1) & ~15);  // (past the last chunk: repeats it, unused)
+    const float* qr = qrow + (size_t)min(tc + r16, a.T - 1) * rstep + g * 4;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      o.q[i] = *reinterpret_cast<const f32x4_t*>(qr + i * 16);
+      o.k[i] = *reinterpret_cast<const f32x4_t*>(qr + D + i * 16);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const size_t t = min(tc + g * 4 + r, a.T - 1);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) o.kt[i][r] = qrow[t * rstep + D + i * 16 + r16];
+      o.v[r] = vcol[t * mixed_w];
+    }
+    const ChunkTable* tab = chunk_tables(a) + (size_t)(tc >> 4) * a.Hv + h;
+    o.inv = *reinterpret_cast<const f32x4_t*>(&tab->inv[r16][g * 4]);
+    o.qk = *reinterpret_cast<const f32x4_t*>(&tab->qk[r16][g * 4]);
+    o.beta = *reinterpret_cast<const f32x4_t*>(&tab->beta[g * 4]);
+    o.dec = *reinterpret_cast<const f32x4_t*>(&tab->dec[g * 4]);
+    o.tail = *reinterpret_cast<const f32x4_t*>(&tab->tail[g * 4]);
+    o.last = tab->dec[15];
+  };
+  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+  auto product = [&](const f32x4_t& x, const f32x4_t& y, f32x4_t acc) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[r], y[r], acc, 0, 0, 0);
+    return acc;
+  };
+  // steps r and r + 1 of a product
+  auto half = [&](const f32x4_t& x, const f32x4_t& y, int r) __attribute__((always_inline)) {
+    const f32x4_t acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[r], y[r], zero, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(x[r + 1], y[r + 1], acc, 0, 0, 0);
+  };
+  // rows of x past token t as zeros
+  auto upto = [&](const f32x4_t& x, int t) __attribute__((always_inline)) {
+    f32x4_t y;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) y[r] = g * 4 + r <= t ? x[r] : 0.f;
+    return y;
+  };
+
+  auto step = [&](const Operands& cur, int c) __attribute__((always_inline)) {
+    // (chains of two and sums in pairs: a chain of eight rounds 32 times at the size of its sum)
+    f32x4_t ks = (half(cur.k[0], S[0], 0) + half(cur.k[0], S[0], 2)) + (half(cur.k[1], S[1], 0) + half(cur.k[1], S[1], 2));
+    f32x4_t qs = (half(cur.q[0], S[0], 0) + half(cur.q[0], S[0], 2)) + (half(cur.q[1], S[1], 0) + half(cur.q[1], S[1], 2));
+    s_part[c & 1][wave][0][lane] = ks;
+    s_part[c & 1][wave][1][lane] = qs;
+    lds_barrier();
+    ks = (s_part[c & 1][0][0][lane] + s_part[c & 1][1][0][lane]) + (s_part[c & 1][2][0][lane] + s_part[c & 1][3][0][lane]);
+    qs = (s_part[c & 1][0][1][lane] + s_part[c & 1][1][1][lane]) + (s_part[c & 1][2][1][lane] + s_part[c & 1][3][1][lane]);
+    f32x4_t rhs;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) rhs[r] = cur.beta[r] * (cur.v[r] - cur.dec[r] * ks[r]);
+    f32x4_t u = rhs + product(cur.inv, rhs, zero), o = zero;
+    // 0 x infinity or NaN: the products' zeros above the diagonal would carry
+    // a later token's non-finite value to an earlier one, so such a chunk
+    // goes token by token (every wavefront holds the same rhs and u)
+    float nf = 0.f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) nf += rhs[r] * 0.f + u[r] * 0.f;
+    if (__builtin_expect(__ballot(nf != 0.f) != 0ull, 0)) {
+      f32x4_t us = zero;
+      for (int t = 0; t < 16; ++t) {
+        const f32x4_t ut = rhs + product(cur.inv, upto(rhs, t - 1), zero);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) us[r] = g * 4 + r == t ? ut[r] : us[r];
+      }
+      u = us;
+      for (int t = 0; t < 16; ++t) {
+        const f32x4_t ot = product(cur.qk, upto(u, t), zero);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[r] = g * 4 + r == t ? ot[r] : o[r];
+      }
+    } else if (wave == (c & 3)) {
+      o = product(cur.qk, u, zero);
+    }
+    if (wave == (c & 3)) {
+      const int t0 = c * 16 + g * 4;
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (t0 + r < a.T)
+          a.ws.core[(size_t)(t0 + r) * a.Hv * D + (size_t)h * D + col] = fmaf(cur.dec[r], qs[r], o[r]);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) S[i] = product(cur.kt[i], cur.tail * u, S[i] * cur.last);
+  };
+  Operands op[3];  // (two chunks in flight: a chunk takes less than a round trip to memory)
+  fetch(op[0], 0);
+  fetch(op[1], 1);
+  const int chunks = (a.T + 15) >> 4;
+  for (int c = 0; c < chunks; c += 3) {
+    fetch(op[2], c + 2);
+    step(op[0], c);
+    if (c + 1 >= chunks) break;
+    fetch(op[0], c + 3);
+    step(op[1], c + 1);
+    if (c + 2 >= chunks) break;
+    fetch(op[1], c + 4);
+    step(op[2], c + 2);
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      store_scalar(a.next_state, a.dt[4], sbase + (size_t)(i * 16 + r) * D, S[i][r]);
 }
 
 // Gated RMSNorm of the scan's outputs, a wavefront per (token, head) of 128:
@@ -1767,8 +2075,16 @@ static int launch_recurrent_output(const RecArgs& ra, const void* out_proj_weigh
   int st;
   // (the scan reads q and k rows of f32 sixteen bytes at a time)
   if (ra.T >= kScanMinTokens && ra.D == 128 && ra.dt[0] == FK_DTYPE_F32 && aligned16(ra.mixed)) {
-    hipLaunchKernelGGL(deltanet_scan_kernel, dim3(ra.Hv, 128 / kScanCols), dim3(256), 0, s, ra);
-    st = check_launch("deltanet_scan_kernel");
+    if (ra.T >= kChunkMinTokens && dn_chunk_bytes(ra.T, ra.Hk, ra.Hv) <= (size_t)ra.T * ra.Hv * ra.D * 6) {
+      hipLaunchKernelGGL(deltanet_chunk_kernel, dim3((ra.T + 15) / 16, ra.Hk), dim3(256), 0, s, ra);
+      st = check_launch("deltanet_chunk_kernel");
+      if (st) return st;
+      hipLaunchKernelGGL(deltanet_chunk_scan_kernel, dim3(ra.Hv, 128 / 16), dim3(256), 0, s, ra);
+      st = check_launch("deltanet_chunk_scan_kernel");
+    } else {
+      hipLaunchKernelGGL(deltanet_scan_kernel, dim3(ra.Hv, 128 / kScanCols), dim3(256), 0, s, ra);
+      st = check_launch("deltanet_scan_kernel");
+    }
     if (st) return st;
     const dim3 ggrid((unsigned)(((size_t)ra.T * ra.Hv + 3) / 4));
     const bool planes = plane_gemm_ok(hidden_size, ra.Hv * ra.D, out_dt);

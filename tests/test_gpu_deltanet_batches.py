@@ -47,7 +47,8 @@ def test_conv_blocks(tokens, kernel_size):
 
 @pytest.mark.parametrize("tokens,qk_heads,value_heads,head_dim", [
     (2, 16, 32, 128), (3, 16, 32, 128), (15, 2, 4, 128), (16, 4, 4, 128), (17, 16, 32, 128), (32, 1, 2, 128), (51, 16, 32, 128),
-    (19, 2, 4, 64),
+    (19, 2, 4, 64), (95, 2, 4, 128), (96, 1, 5, 128), (97, 2, 4, 128), (112, 16, 32, 128), (127, 1, 2, 128), (100, 4, 4, 128),
+    (250, 2, 4, 128),
 ])
 @pytest.mark.parametrize("hidden", [256, 250])  # 250: the general output projection
 def test_recurrence_chunks(tokens, qk_heads, value_heads, head_dim, hidden):
@@ -86,6 +87,35 @@ def test_recurrence_chunks(tokens, qk_heads, value_heads, head_dim, hidden):
     # its decay and delta forget again
     assert float((state.cpu().double() - s).norm() / s.norm()) < 2e-6
     assert float((update.cpu().double() - ref).norm() / ref.norm()) < 4e-6
+
+
+@pytest.mark.parametrize("what", ["value", "key", "beta"])
+def test_recurrence_keeps_a_non_finite_token_from_earlier_ones(what):
+    """Rows before a non-finite token (inside a chunk of 16) are what they are without it, other heads' states too."""
+
+    tokens, bad, gen = 120, 101, torch.Generator().manual_seed(1)
+    mixed, z = _randn(gen, (tokens, 2 * 2 * 128 + 512)).cuda(), _randn(gen, (tokens, 512)).cuda()
+    a, b, state = _randn(gen, (tokens, 4)).cuda(), _randn(gen, (tokens, 4)).cuda(), _randn(gen, (4, 128, 128), 0.1).cuda()
+    rest = (_randn(gen, (256, 512), 0.02, torch.bfloat16).cuda(), _randn(gen, (128,)).cuda(), _randn(gen, (4,), 0.5).cuda(),
+            _randn(gen, (4,), 0.5).cuda())
+    run = lambda: hip.hip_qwen36_batched_deltanet_recurrent_output(  # noqa: E731
+        mixed, z, a, b, state, *rest, qk_heads=2, value_heads=4, head_dim=128)
+    update, after = run()
+    if what == "value":
+        mixed[bad, 512 + 3] = float("inf")  # head 0, column 3
+    elif what == "key":
+        mixed[bad, 256 + 5] = float("nan")  # qk head 0: value heads 0 and 1
+    else:
+        b[bad, 0] = float("nan")
+    update2, after2 = run()
+    # (that chunk goes token by token: a delta may round once more or less, 2^-24 of values below 4)
+    near = lambda x, y: torch.allclose(x, y, rtol=1e-6, atol=4e-6)  # noqa: E731
+    assert near(update2[:bad], update[:bad])
+    assert not torch.isfinite(update2[bad]).any() and not torch.isfinite(after2[0]).all()
+    assert torch.equal(after2[2:], after[2:])
+    if what == "value":  # the state's other columns too
+        keep = [c for c in range(128) if c != 3]
+        assert near(after2[0][:, keep], after[0][:, keep]) and torch.equal(after2[1], after[1])
 
 
 @pytest.mark.parametrize("tokens,conv_dtype", [(9, torch.bfloat16), (16, torch.bfloat16), (33, torch.float32),
