@@ -146,11 +146,16 @@ __global__ __launch_bounds__(256) void attn_prompt_prep_kernel(PromptArgs a) {
 //   O^T = V^T P^T: step q takes position 4 (l / 16) + q, which is where the
 //     lane's probability already is; row r of value tile (g, i) is dim
 //     64 g + 4 r + i
+// Products of 16 dims (scores) and of a tile's 16 positions (values) start
+// from zero and are added by the VALU, the scores' in pairs: summed inside the
+// MFMAs throughout (chains of 128 products, and the running sum of the values)
+// the calls' error against 64 bits was 6.3e-7 to 9.1e-7 at 300 to 3,000
+// positions, where it is 3.1e-7 to 4.3e-7 (the VALU dot products that this
+// replaced: 3.3e-7 to 4.4e-7), for 1 to 2% of a call's time.
 // The 16-byte chunks of a tile row are XOR-swizzled by the row.  Bound by the
 // fp32 MFMAs (128 of 32 cycles a wavefront and tile) and, between them, the
-// tile's chain of maximum, exponentials and barrier, which the second
-// workgroup of the CU covers in part: 200 rows behind 1,000 positions, 3.6
-// GFLOP, take 73 us, a third of the matrix rate.
+// tile's chain of sums, maximum, exponentials and barrier, which the second
+// workgroup of the CU covers in part.
 template <bool CBF>
 __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(PromptArgs a) {
   constexpr int hd = kPromptHd, CH = hd / 4;
@@ -229,9 +234,24 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(PromptArgs a) {
       s_v[b][r][lane ^ r] = v4;
     }
   };
+  // the swizzled chunks, up to multiples of 16 (four addresses each, not one per read)
+  int kx[4], vx[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    kx[i] = (i * 4 + g4) ^ n;  // chunk 4 J + l / 16 of key l % 16: 16 (J / 4) + kx[J % 4]
+    vx[i] = n ^ (g4 * 4 + i);  // chunk 16 g + l % 16 of key 4 (l / 16) + i: 16 g + vx[i]
+  }
+  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+  // four steps of a product, from zero
+  auto product = [&](const f32x4_t& x, const f32x4_t& y) __attribute__((always_inline)) {
+    f32x4_t c = zero;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_16x16x4f32(x[e], y[e], c, 0, 0, 0);
+    return c;
+  };
   f32x4_t o[16];
 #pragma unroll
-  for (int d = 0; d < 16; ++d) o[d] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int d = 0; d < 16; ++d) o[d] = zero;
   float m = -INFINITY, l = 0.f;
 
   fetch(p_lo);
@@ -239,42 +259,45 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(PromptArgs a) {
   __syncthreads();
   for (int p0 = p_lo, b = 0; p0 < p_hi; p0 += kPromptTile, b ^= 1) {
     fetch(p0 + kPromptTile);
-    f32x4_t s4[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};  // two sums: an MFMA needs the one before its own last
-#pragma unroll
-    for (int J = 0; J < 16; ++J) {
-      const f32x4_t k4 = s_k[b][n][(J * 4 + g4) ^ n];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) s4[e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[e], q[J][e], s4[e & 1], 0, 0, 0);
+    f32x4_t s4;  // (the products of 16 dims each, added in pairs)
+    {
+      auto dims16 = [&](int J) __attribute__((always_inline)) { return product(s_k[b][n][(J >> 2) * 16 + kx[J & 3]], q[J]); };
+      auto dims64 = [&](int J) __attribute__((always_inline)) {
+        const f32x4_t lo = dims16(J) + dims16(J + 1);
+        return lo + (dims16(J + 2) + dims16(J + 3));
+      };
+      const f32x4_t lo = dims64(0) + dims64(4);
+      s4 = lo + (dims64(8) + dims64(12));
     }
-    float p[4], mx = -INFINITY;
+    f32x4_t p;
+    float mx = -INFINITY;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int at = p0 + g4 * 4 + i;
-      p[i] = at <= pos && at < p_hi ? s4[0][i] + s4[1][i] : -INFINITY;
+      p[i] = at <= pos && at < p_hi ? s4[i] : -INFINITY;
       mx = fmaxf(mx, p[i]);
     }
     mx = fmaxf(mx, __uint_as_float(xor16_u32(__float_as_uint(mx))));
     mx = fmaxf(mx, __uint_as_float(xor32_u32(__float_as_uint(mx))));
     const float mn = fmaxf(m, mx);
     const float f = m == -INFINITY ? 0.f : __expf(m - mn);  // (nothing summed yet: 0)
-    l *= f;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      p[i] = p[i] == -INFINITY ? 0.f : __expf(p[i] - mn);
-      l += p[i];
-    }
+    for (int i = 0; i < 4; ++i) p[i] = p[i] == -INFINITY ? 0.f : __expf(p[i] - mn);
+    l = fmaf(l, f, (p[0] + p[1]) + (p[2] + p[3]));
     m = mn;
 #pragma unroll
-    for (int d = 0; d < 16; ++d) o[d] *= f;
+    for (int g = 0; g < 4; ++g) {
+      f32x4_t v4[4];
 #pragma unroll
-    for (int g = 0; g < 4; ++g)
+      for (int i = 0; i < 4; ++i) v4[i] = s_v[b][g4 * 4 + i][g * 16 + vx[i]];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int key = g4 * 4 + i;
-        const f32x4_t v4 = s_v[b][key][(g * 16 + n) ^ key];
+      for (int e = 0; e < 4; ++e) {
+        const f32x4_t c = product(f32x4_t{v4[0][e], v4[1][e], v4[2][e], v4[3][e]}, p);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o[g * 4 + e] = __builtin_amdgcn_mfma_f32_16x16x4f32(v4[e], p[i], o[g * 4 + e], 0, 0, 0);
+        for (int r = 0; r < 4; ++r) o[g * 4 + e][r] = fmaf(o[g * 4 + e][r], f, c[r]);
+        asm volatile("" : "+v"(o[g * 4 + e]));  // (sunk into the loop's next block, the updates would keep every product)
       }
+    }
     stage(b ^ 1, p0 + kPromptTile);  // (past the last tile: not read)
     __syncthreads();
   }

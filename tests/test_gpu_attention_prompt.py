@@ -84,6 +84,34 @@ def test_prompt_rows(tokens, start, hidden, heads, kvh, x_dtype, cache_dtype, in
     assert torch.equal(update, again[0])
 
 
+def _error(seed, tokens, start, hidden, heads, kvh, cache_dtype):
+    """Relative error against float64 without rotation (whose 32-bit angles are
+    the largest part of it otherwise) and with q norm weights near 2 (scores of
+    a few units, as a trained model's)."""
+
+    x, kc, vc, w = _inputs(seed, tokens, hidden, heads, kvh, start + tokens, torch.float32, cache_dtype)
+    w["q_norm_weight"] = (w["q_norm_weight"].float() + 1.0).bfloat16()
+    got = hip.hip_qwen36_batched_attention_decode(
+        x, kc, vc, *w.values(), start_position=start, attention_heads=heads, kv_heads=kvh, rope_dim=0)[0]
+    ref, _, _ = _reference(x, kc, vc, w, start, heads, kvh, 0, 1e4, True)
+    return float((got.double() - ref).norm() / ref.norm())
+
+
+# A score is a sum of 256 products, whose roundings all reach the output.  In
+# short chains added in pairs, as the dot products of few rows are (4 products
+# and 6 levels), the variance is about 8 to 12 squared roundings of the score;
+# in two chains of 128 products it is 64.  Measured: 3.1e-7 to 4.6e-7 and
+# 6.1e-7 to 9.9e-7; the bound lies between them.
+@pytest.mark.parametrize("tokens,start,hidden,heads,kvh,cache_dtype", [
+    (8, 1000, 512, 8, 1, torch.float32),
+    (32, 3000, 512, 16, 2, torch.bfloat16),
+    (200, 1000, 2048, 16, 2, torch.float32),
+])
+def test_prompt_sums_are_as_exact_as_dot_products(tokens, start, hidden, heads, kvh, cache_dtype):
+    errs = [_error(seed, tokens, start, hidden, heads, kvh, cache_dtype) for seed in range(3)]
+    assert sum(errs) / 3 < 5.2e-7, errs
+
+
 # step calls with long chunks of positions per workgroup (64, 32, 21 and 16
 # chunks for 1 to 4 tokens): the last chunk length of the loop over tiles (48)
 # and the first past it, tiles of 64 positions with every kind of remainder,
