@@ -1117,8 +1117,11 @@ __global__ __launch_bounds__(kAsThreads) void attn_step_kernel(AttnStepArgs a) {
       // tile's rows in flight (two register sets).  The loop over tiles below
       // is bound by VALU issue (a dot product per head and position, one
       // wavefront pair per SIMD) and by a memory round trip per 24 positions:
-      // 12,000 positions took 35.8 us a step with it (bf16 cache), 30.5 here;
-      // 4 tokens 86.1 -> 59.3.
+      // 12,000 positions took 36.8 us a step with it (bf16 cache), 31.7 here;
+      // 4 tokens 88.2 -> 64.1.  Products start from zero every four dims (and
+      // keys), as that loop's do: in chains of eight, with the values added to
+      // the running sum inside the MFMAs, the error against 64 bits was 5 to
+      // 10% larger, for 0.3 us (4 tokens 1.4) less.
       const int blk = lane >> 2, hc = lane & 3;
       float4 qv[4];
 #pragma unroll
@@ -1127,16 +1130,15 @@ __global__ __launch_bounds__(kAsThreads) void attn_step_kernel(AttnStepArgs a) {
       for (int u = 0; u < 4; ++u) lo[u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
       // four keys: their scores for the lane's head (all blocks added)
       auto scores4 = [&](const float4 (&k4)[4], f32x4_t& out) __attribute__((always_inline)) {
-        f32x4_t s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
+        f32x4_t su[4];  // chains of four products, added in pairs
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-          f32x4_t& su = u & 1 ? s1 : s0;
-          su = __builtin_amdgcn_mfma_f32_4x4x1f32(k4[u].x, qv[u].x, su, 0, 0, 0);
-          su = __builtin_amdgcn_mfma_f32_4x4x1f32(k4[u].y, qv[u].y, su, 0, 0, 0);
-          su = __builtin_amdgcn_mfma_f32_4x4x1f32(k4[u].z, qv[u].z, su, 0, 0, 0);
-          su = __builtin_amdgcn_mfma_f32_4x4x1f32(k4[u].w, qv[u].w, su, 0, 0, 0);
+          su[u] = __builtin_amdgcn_mfma_f32_4x4x1f32(k4[u].x, qv[u].x, f32x4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+          su[u] = __builtin_amdgcn_mfma_f32_4x4x1f32(k4[u].y, qv[u].y, su[u], 0, 0, 0);
+          su[u] = __builtin_amdgcn_mfma_f32_4x4x1f32(k4[u].z, qv[u].z, su[u], 0, 0, 0);
+          su[u] = __builtin_amdgcn_mfma_f32_4x4x1f32(k4[u].w, qv[u].w, su[u], 0, 0, 0);
         }
-        out = s0 + s1;
+        out = (su[0] + su[1]) + (su[2] + su[3]);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           float v = out[r];
@@ -1153,18 +1155,28 @@ __global__ __launch_bounds__(kAsThreads) void attn_step_kernel(AttnStepArgs a) {
 #pragma unroll
         for (int i = 0; i < N; ++i) mx = fmaxf(mx, sc[i >> 2][i & 3]);
         const float f = lm == -INFINITY ? 0.f : __expf(lm - mx);
-        ll *= f;
+        float es[4] = {0.f, 0.f, 0.f, 0.f};
+        f32x4_t c[4];  // the values' sums over the keys, from zero, four keys at a time
 #pragma unroll
-        for (int u = 0; u < 4; ++u) lo[u] *= f;
+        for (int h = 0; h < N; h += 4) {
+          f32x4_t ch[4];
 #pragma unroll
-        for (int i = 0; i < N; ++i) {
-          const float s = sc[i >> 2][i & 3], p = s == -INFINITY ? 0.f : __expf(s - mx);
-          ll += p;
-          lo[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(v4[i].x, p, lo[0], 0, 0, 0);
-          lo[1] = __builtin_amdgcn_mfma_f32_4x4x1f32(v4[i].y, p, lo[1], 0, 0, 0);
-          lo[2] = __builtin_amdgcn_mfma_f32_4x4x1f32(v4[i].z, p, lo[2], 0, 0, 0);
-          lo[3] = __builtin_amdgcn_mfma_f32_4x4x1f32(v4[i].w, p, lo[3], 0, 0, 0);
+          for (int i = 0; i < 4; ++i) {
+            const float s = sc[h >> 2][i], p = s == -INFINITY ? 0.f : __expf(s - mx);
+            es[i] += p;
+            const float v[4] = {v4[h + i].x, v4[h + i].y, v4[h + i].z, v4[h + i].w};
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+              ch[u] = __builtin_amdgcn_mfma_f32_4x4x1f32(v[u], p, i ? ch[u] : f32x4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+          }
+#pragma unroll
+          for (int u = 0; u < 4; ++u) c[u] = h ? c[u] + ch[u] : ch[u];
         }
+        ll = fmaf(ll, f, (es[0] + es[1]) + (es[2] + es[3]));
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) lo[u][r] = fmaf(lo[u][r], f, c[u][r]);
         lm = mx;
       };
       auto tile = [&](const Row4<CBF>(&kr)[2][4], const Row4<CBF>(&vr)[8], int pt) __attribute__((always_inline)) {

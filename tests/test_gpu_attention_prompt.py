@@ -84,13 +84,13 @@ def test_prompt_rows(tokens, start, hidden, heads, kvh, x_dtype, cache_dtype, in
     assert torch.equal(update, again[0])
 
 
-def _error(seed, tokens, start, hidden, heads, kvh, cache_dtype):
+def _error(seed, tokens, start, hidden, heads, kvh, cache_dtype, q_norm=1.0):
     """Relative error against float64 without rotation (whose 32-bit angles are
-    the largest part of it otherwise) and with q norm weights near 2 (scores of
-    a few units, as a trained model's)."""
+    the largest part of it otherwise) and with q norm weights near 1 + q_norm
+    (scores of a few units, as a trained model's)."""
 
     x, kc, vc, w = _inputs(seed, tokens, hidden, heads, kvh, start + tokens, torch.float32, cache_dtype)
-    w["q_norm_weight"] = (w["q_norm_weight"].float() + 1.0).bfloat16()
+    w["q_norm_weight"] = (w["q_norm_weight"].float() + q_norm).bfloat16()
     got = hip.hip_qwen36_batched_attention_decode(
         x, kc, vc, *w.values(), start_position=start, attention_heads=heads, kv_heads=kvh, rope_dim=0)[0]
     ref, _, _ = _reference(x, kc, vc, w, start, heads, kvh, 0, 1e4, True)
@@ -132,6 +132,15 @@ def test_prompt_sums_are_as_exact_as_dot_products(tokens, start, hidden, heads, 
 ])
 def test_step_of_long_chunks(tokens, start, hidden, heads, kvh, cache_dtype):
     test_prompt_rows(tokens, start, hidden, heads, kvh, torch.float32, cache_dtype, True)
+
+
+def test_long_chunk_sums_are_as_exact_as_the_loop_over_tiles():
+    """Scores in chains of four products and values in sums of four positions,
+    as the loop over tiles adds them (4.96e-7 here): 5.10e-7.  In chains of
+    eight, with the values on the running sum: 5.50e-7."""
+
+    errs = [_error(seed, 4, 12000, 512, 16, 2, torch.float32, 3.0) for seed in range(8)]
+    assert sum(errs) / 8 < 5.3e-7, errs
 
 
 def test_rows_see_no_later_row():
