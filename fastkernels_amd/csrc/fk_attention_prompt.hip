@@ -47,6 +47,7 @@ struct PromptArgs {
   float theta_log2, eps;
   float* q_rot;  // [T, heads, hd] normalised, rotated, times hd^-1/2
   float* k_rot;  // [T, kvh, hd]
+  int* v_bad;    // [T, kvh] whether the row's values hold an infinity or NaN
   float* stat;   // [T, heads, nc, 2] chunk maximum and sum
   float* acc;    // [T, heads, nc, hd] chunk's weighted values
   int nc, chunk; // chunks of positions
@@ -119,6 +120,9 @@ __global__ __launch_bounds__(256) void attn_prompt_prep_kernel(PromptArgs a) {
   *reinterpret_cast<float4*>(a.k_rot + ((size_t)t * a.kvh + j) * hd + lane * 4) = make_float4(y[0], y[1], y[2], y[3]);
   if (start < 0) return;  // no cache access
   const float4 v4 = *reinterpret_cast<const float4*>(a.v + ((size_t)t * a.kvh + j) * hd + lane * 4);
+  const bool bad = __ballot(!(fabsf(v4.x) < INFINITY && fabsf(v4.y) < INFINITY && fabsf(v4.z) < INFINITY &&
+                              fabsf(v4.w) < INFINITY)) != 0ull;
+  if (lane == 0) a.v_bad[t * a.kvh + j] = bad;
   const size_t o = ((size_t)(start + t) * a.kvh + j) * hd + lane * 4;
   if constexpr (CBF) {
     // (the same rounding as store_scalar's, NaN kept)
@@ -215,22 +219,20 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(PromptArgs a) {
       }
     }
   };
-  // A tile holds positions that some of its queries do not see: their
+  // A tile may hold positions that some of its queries do not see: their
   // probabilities are 0, which an infinity or NaN among the values (a later
-  // token's) would still turn into NaN.  Such a value of the call's own rows
-  // is staged as 0 and its key as NaN: the queries that see the position get
-  // NaN, the others nothing.
+  // token's) would still turn into NaN.  Such values of the call's own rows
+  // are staged as 0; attn_prompt_merge_kernel adds them for the queries that
+  // see them.
   auto stage = [&](int b, int p0) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int r = wave + 4 * i;
-      f32x4_t k4 = rk[i], v4 = rv[i];
-      const bool bad = min(p0 + r, p_hi - 1) >= start && !(fabsf(v4[0]) < INFINITY && fabsf(v4[1]) < INFINITY &&
-                                                           fabsf(v4[2]) < INFINITY && fabsf(v4[3]) < INFINITY);
-      k4[0] = bad ? __builtin_nanf("") : k4[0];
+      f32x4_t v4 = rv[i];
+      const bool own = min(p0 + r, p_hi - 1) >= start;  // (uniform)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v4[e] = bad ? 0.f : v4[e];
-      s_k[b][r][lane ^ r] = k4;
+      for (int e = 0; e < 4; ++e) v4[e] = own && !(fabsf(v4[e]) < INFINITY) ? 0.f : v4[e];
+      s_k[b][r][lane ^ r] = rk[i];
       s_v[b][r][lane ^ r] = v4;
     }
   };
@@ -316,7 +318,8 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(PromptArgs a) {
 }
 
 // A wavefront per (token, head): the chunks that the token reaches, against
-// the largest chunk maximum in chunk order, the output gate, three bf16 terms.
+// the largest chunk maximum in chunk order, the own values that are not
+// finite, the output gate, three bf16 terms.
 __global__ __launch_bounds__(256) void attn_prompt_merge_kernel(PromptArgs a) {
   constexpr int hd = kPromptHd;
   const int lane = threadIdx.x & 63;
@@ -342,6 +345,21 @@ __global__ __launch_bounds__(256) void attn_prompt_merge_kernel(PromptArgs a) {
     o.z = fmaf(v.z, f, o.z);
     o.w = fmaf(v.w, f, o.w);
   }
+  // the call's own values that are not finite, which the chunks summed as 0
+  const int j = (int)(row - (long long)t * a.heads) / (a.heads / a.kvh);
+  for (int u0 = 0; start >= 0 && u0 <= t; u0 += kWave) {
+    uint64_t rows = __ballot(u0 + lane <= t && a.v_bad[(size_t)min(u0 + lane, t) * a.kvh + j] != 0);
+    for (; rows; rows &= rows - 1) {
+      const size_t at = ((size_t)(u0 + __builtin_ctzll(rows)) * a.kvh + j) * hd + lane * 4;
+      const float4 q4 = *reinterpret_cast<const float4*>(a.q_rot + (size_t)row * hd + lane * 4);
+      const float4 k4 = *reinterpret_cast<const float4*>(a.k_rot + at), v4 = *reinterpret_cast<const float4*>(a.v + at);
+      const float p = __expf(wave_sum((q4.x * k4.x + q4.y * k4.y) + (q4.z * k4.z + q4.w * k4.w)) - M);
+      o.x += fabsf(v4.x) < INFINITY ? 0.f : p * v4.x;
+      o.y += fabsf(v4.y) < INFINITY ? 0.f : p * v4.y;
+      o.z += fabsf(v4.z) < INFINITY ? 0.f : p * v4.z;
+      o.w += fabsf(v4.w) < INFINITY ? 0.f : p * v4.w;
+    }
+  }
   const float4 gate = *reinterpret_cast<const float4*>(a.qg + (size_t)row * 2 * hd + hd + lane * 4);
   const float y[4] = {poison_if(start < 0, (o.x / L) * sigmoid(gate.x)), poison_if(start < 0, (o.y / L) * sigmoid(gate.y)),
                       poison_if(start < 0, (o.z / L) * sigmoid(gate.z)), poison_if(start < 0, (o.w / L) * sigmoid(gate.w))};
@@ -362,6 +380,7 @@ __global__ void attn_prompt_advance_kernel(int* start, int T, int max_pos) {
 
 struct PromptWs {
   float *qg, *k, *v, *q_rot, *k_rot, *stat, *acc, *part;
+  int* v_bad;
   uint16_t* planes;
   size_t part_bytes;
 };
@@ -387,6 +406,7 @@ static size_t prompt_ws_layout(int T, int heads, int kvh, char* base, PromptWs* 
   ws->v = floats(kv);
   ws->q_rot = floats(q);
   ws->k_rot = floats(kv);
+  ws->v_bad = reinterpret_cast<int*>(take((size_t)T * kvh * 4));
   ws->stat = floats((size_t)T * heads * nc * 2);
   ws->acc = floats(q * nc);
   ws->planes = reinterpret_cast<uint16_t*>(take(q * 6));
@@ -437,6 +457,7 @@ int launch_attn_prompt(const AttnPromptCall& p, void* workspace, hipStream_t s) 
   a.eps = p.qk_eps;
   a.q_rot = ws.q_rot;
   a.k_rot = ws.k_rot;
+  a.v_bad = ws.v_bad;
   a.stat = ws.stat;
   a.acc = ws.acc;
   a.planes = ws.planes;

@@ -156,6 +156,24 @@ def test_rows_see_no_later_row():
     assert bool(got[21:].isnan().all())
 
 
+@pytest.mark.parametrize("tokens,start,row", [(8, 1000, 0), (8, 30, 7), (40, 100, 17), (70, 0, 69)])
+def test_infinite_value_of_the_call_stays_infinite(tokens, start, row):
+    """One value of one row overflows: the rows that see it get that infinity,
+    in that dim alone, and the rows before it nothing."""
+
+    x, kc, vc, w = _inputs(4, tokens, 512, 8, 2, start + tokens, torch.float32, torch.float32)
+    x[:, 3], x[row, 3] = 0.0, 5.0
+    w["norm_weight"][3] = 0.0
+    w["v_proj_weight"][5], w["v_proj_weight"][5, 3] = 0.0, 3e38  # kv head 0, dim 5
+    w["out_proj_weight"][:, 5:4 * 256:256] = 0.02               # of its four query heads: the infinities add up
+    kw = dict(start_position=start, attention_heads=8, kv_heads=2, rope_dim=64)
+    got, _, v = hip.hip_qwen36_batched_attention_decode(x, kc, vc, *w.values(), **kw)
+    assert bool(v[start + row, 0, 5].isposinf()) and int((~v.isfinite()).sum()) == 1
+    assert bool(got[row:].isposinf().all())
+    w["v_proj_weight"][5, 3] = 0.0
+    assert torch.equal(got[:row], hip.hip_qwen36_batched_attention_decode(x, kc, vc, *w.values(), **kw)[0][:row])
+
+
 @pytest.mark.parametrize("tokens", [8, 32])
 def test_device_position_advances_and_is_checked(tokens):
     x, kc, vc, w = _inputs(7, tokens, 2048, 16, 2, 4 * tokens, torch.bfloat16, torch.float32)
