@@ -1195,6 +1195,11 @@ __global__ __launch_bounds__(kAsThreads) void attn_step_kernel(AttnStepArgs a) {
         }
 #pragma unroll
         for (int i = 0; i < 8; ++i) v4[i] = vr[i].f4();
+        if (pw + 8 > pc_hi) {  // (uniform) the repeated rows' values, which an infinity would turn 0 x v to NaN with
+#pragma unroll
+          for (int i = 1; i < 8; ++i)
+            if (pw + i >= pc_hi) v4[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
         fold(sc, v4, std::integral_constant<int, 8>{});
       };
       if (wave == kAsWaves - 1 && n_own > 0) {  // the step's own positions (at most four)
@@ -1208,6 +1213,7 @@ __global__ __launch_bounds__(kAsThreads) void attn_step_kernel(AttnStepArgs a) {
         for (int r = 0; r < 4; ++r) {
           sc[0][r] = r < n_own ? sc[0][r] : -INFINITY;
           v4[r] = *reinterpret_cast<const float4*>(s_vn + min(r, n_own - 1) * hd + lane * 4);
+          if (r >= n_own) v4[r] = make_float4(0.f, 0.f, 0.f, 0.f);
         }
         fold(sc, v4, std::integral_constant<int, 4>{});
       }

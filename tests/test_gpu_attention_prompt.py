@@ -174,6 +174,18 @@ def test_infinite_value_of_the_call_stays_infinite(tokens, start, row):
     assert torch.equal(got[:row], hip.hip_qwen36_batched_attention_decode(x, kc, vc, *w.values(), **kw)[0][:row])
 
 
+# the last cached position before the step's own (one that loads past the
+# chunk repeat), and an inner one, for calls of few and of many rows
+@pytest.mark.parametrize("tokens,start,at", [(1, 4095, 4094), (1, 4095, 70), (3, 3071, 3070), (4, 12000, 11999), (8, 1000, 999), (33, 900, 31)])
+def test_infinite_cached_value_stays_infinite(tokens, start, at):
+    x, kc, vc, w = _inputs(5, tokens, 512, 16, 2, start + tokens, torch.float32, torch.float32)
+    vc[at, 0, 5] = float("inf")
+    w["out_proj_weight"][:, 5:8 * 256:256] = 0.02
+    got = hip.hip_qwen36_batched_attention_decode(
+        x, kc, vc, *w.values(), start_position=start, attention_heads=16, kv_heads=2, rope_dim=64)[0]
+    assert bool(got.isposinf().all())
+
+
 @pytest.mark.parametrize("tokens", [8, 32])
 def test_device_position_advances_and_is_checked(tokens):
     x, kc, vc, w = _inputs(7, tokens, 2048, 16, 2, 4 * tokens, torch.bfloat16, torch.float32)
