@@ -149,7 +149,8 @@ __global__ __launch_bounds__(64 * WN * WM, OCC) void token_gemm_kernel(GemmArgs 
           v[q] *= a.off + g[q];
         }
         ss[p] = real ? ss[p] + sq : ss[p];
-        split3_8(v, pr[ux][p][0], pr[ux][p][1], pr[ux][p][2]);
+        // (an infinity makes its row's scale 0 and the row NaN either way)
+        split3_8<false>(v, pr[ux][p][0], pr[ux][p][1], pr[ux][p][2]);
       }
       staged += kGemmBK;
     }

@@ -80,6 +80,21 @@ def test_one_expert_takes_every_pair():
     assert float((out.double() - ref).norm() / ref.norm()) < 1e-6
 
 
+def test_values_past_the_bf16_range():
+    """fp32 hidden states above the largest bf16 (3.39e38), against weights that bring them back into range."""
+
+    gen = torch.Generator().manual_seed(11)
+    gu, dn = _randn(gen, (8, 512, 512), 0.02), _randn(gen, (8, 512, 256), 0.02)
+    x = _randn(gen, (100, 512), 1.0, torch.float32)
+    x[::7, 9] = 3.4e38
+    gu[:, :, 9] = 1e-38
+    ids = torch.rand((100, 8), generator=gen).topk(2, dim=-1).indices.cuda()
+    w = torch.rand((100, 2), generator=gen).cuda()
+    out = hip.hip_qwen36_batched_routed_experts_decode(x, ids, w, gu, dn)
+    ref = _reference(x, ids, w, gu, dn)
+    assert float((out.double() - ref).norm() / ref.norm()) < 1e-6
+
+
 @pytest.mark.parametrize("pairs,experts", [(1, 1), (63, 3), (64, 256), (65, 2), (1023, 7), (1030, 1024), (4096, 256), (4096, 1)])
 def test_routing_tables(pairs, experts):
     from oracle import qwen36 as oracle

@@ -77,3 +77,17 @@ def test_large_and_non_finite_tokens():
         assert bool(o[3].isnan().all()) and bool(o[5].isnan().all()) and bool(f[0].isnan().all()) and bool(f[2].isnan().all())
     keep = [t for t in range(20) if t not in (3, 5)]
     _check([o[keep] for o in outs], x[keep], norm, w)
+
+
+@pytest.mark.parametrize("tokens", [4, 40, 200])
+def test_values_past_the_bf16_range(tokens):
+    """A finite value above the largest bf16 (3.39e38) is no infinity: its
+    token's norm scale is 0 (the squares overflow), and so are its products."""
+
+    gen = torch.Generator().manual_seed(5)
+    x, norm = _randn(gen, (tokens, 512), 1.0, torch.float32), _randn(gen, (512,), 0.1)
+    norm[7] = 0.0
+    x[2, 7], x[3, 7] = 3.4e38, -3.4028234e38
+    w = [_randn(gen, (n, 512), 0.02) for n in (64, 32, 16, 16)]
+    for out in hip.hip_qwen36_batched_deltanet_project(x, norm, *w):
+        assert bool((out[2:4] == 0).all()) and bool(out.isfinite().all())
