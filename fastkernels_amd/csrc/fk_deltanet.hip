@@ -927,6 +927,7 @@ __global__ __launch_bounds__(256) void deltanet_chunk_scan_kernel(RecArgs a) {
         if (t0 + r < a.T)
           a.ws.core[(size_t)(t0 + r) * a.Hv * D + (size_t)h * D + col] = fmaf(cur.dec[r], qs[r], o[r]);
     }
+    if (c * 16 + 16 > a.T) u = upto(u, a.T - 1 - c * 16);  // (beta 0 x a last token's infinity is NaN past the end)
 #pragma unroll
     for (int i = 0; i < 2; ++i) S[i] = product(cur.kt[i], cur.tail * u, S[i] * cur.last);
   };

@@ -118,6 +118,23 @@ def test_recurrence_keeps_a_non_finite_token_from_earlier_ones(what):
         assert near(after2[0][:, keep], after[0][:, keep]) and torch.equal(after2[1], after[1])
 
 
+@pytest.mark.parametrize("tokens", [20, 97, 100, 112])
+def test_recurrence_infinite_last_value(tokens):
+    """An infinite value of the last token leaves its column of the state
+    infinite (k times it), also where the last chunk of 16 is not full."""
+
+    gen = torch.Generator().manual_seed(2)
+    mixed, z = _randn(gen, (tokens, 2 * 2 * 128 + 512)), _randn(gen, (tokens, 512))
+    mixed[-1, 512 + 3] = float("inf")  # head 0, column 3
+    a, b, state = _randn(gen, (tokens, 4)), _randn(gen, (tokens, 4)), _randn(gen, (4, 128, 128), 0.1)
+    rest = (_randn(gen, (256, 512), 0.02, torch.bfloat16), _randn(gen, (128,)), _randn(gen, (4,), 0.5), _randn(gen, (4,), 0.5))
+    _, after = hip.hip_qwen36_batched_deltanet_recurrent_output(
+        *(t.cuda() for t in (mixed, z, a, b, state, *rest)), qk_heads=2, value_heads=4, head_dim=128)
+    column = after[0, :, 3].cpu()
+    assert bool(column.isinf().all()) and torch.equal(column > 0, mixed[-1, 256:384] > 0)
+    assert int((~after.isfinite()).sum()) == 128
+
+
 @pytest.mark.parametrize("tokens,conv_dtype", [(9, torch.bfloat16), (16, torch.bfloat16), (33, torch.float32),
                                                (64, torch.bfloat16), (4, torch.float32)])
 def test_step_equals_staged_operators(tokens, conv_dtype):
