@@ -195,7 +195,7 @@ __global__ __launch_bounds__(256) void attn_split_kernel(AttnArgs a) {
   const uint32_t qnw = elem_word(a.qn_w, a.qn_dt, dq);
   const uint32_t knw = elem_word(a.kn_w, a.kn_dt, dq);
   const int start = a.start_dev ? *a.start_dev : a.start;
-  if (start < 0 || start + a.T > a.max_pos) {
+  if (!positions_in_cache(start, a.T, a.max_pos)) {
     // a run-time position past the cache: no cache access, NaN outputs
     if (c == 0 && in)
       for (int g = 0; g < G; ++g) a.gated[(size_t)t * qw + (size_t)(hb + g) * hd + tid] = __builtin_nanf("");
@@ -442,7 +442,7 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnMergeArgs a) {
   const int dc = min(d, kAttnMaxChunks - 1);
   const float mc = base[(size_t)dc * (hd + 2)], lc = base[(size_t)dc * (hd + 2) + 1];
   const int start = a.start_dev ? *a.start_dev : a.start;
-  if (start < 0 || start + a.T > a.max_pos) return;  // the split kernel wrote NaN outputs
+  if (!positions_in_cache(start, a.T, a.max_pos)) return;  // the split kernel wrote NaN outputs
   const int pos = start + t, nc = (pos + a.chunk) / a.chunk;
   if (nc == 1) return;  // the split kernel wrote the gated output itself
   if (d < kAttnMaxChunks) {
@@ -626,7 +626,7 @@ __global__ __launch_bounds__(256) void attn_out_kernel(AttnOutArgs a) {
   // step would pass the cache (NaN update) stays, and the error word says so
   if (a.advance && blockIdx.x == 0 && threadIdx.x == 0) {
     const int s0 = *a.advance;
-    if (s0 >= 0 && s0 + a.T <= a.max_pos) *a.advance = s0 + a.T;
+    if (positions_in_cache(s0, a.T, a.max_pos)) *a.advance = s0 + a.T;
     else __hip_atomic_fetch_or(a.err, FK_DEVICE_ERR_POSITION, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
@@ -947,7 +947,7 @@ __global__ __launch_bounds__(kAsThreads) void attn_step_kernel(AttnStepArgs a) {
       tag = wl.tag;
       plim = wl.poll;
       start = (int)s_hdr[3];
-      bad_pos = start < 0 || start + T > a.max_pos;
+      bad_pos = !positions_in_cache(start, T, a.max_pos);
       apos = start + at;
       an = bad_pos ? 0 : apos + 1;
       const int aC = (an + nch - 1) / nch;
@@ -1695,9 +1695,9 @@ int fk_attention_decode(const void* hidden, int hidden_dtype, const void* norm_w
   int st = check_attn_shape(tokens, hidden_size, heads, kv_heads, head_dim, rope_dim);
   if (st) return st;
   if (max_positions < 1) return fail(FK_ERR_INVALID, "max_positions must be positive");
-  if (!start_position_device && (start_position < 0 || start_position + tokens > max_positions))
-    return fail(FK_ERR_INVALID, "decode positions [%d, %d) exceed the cache length %d", start_position,
-                start_position + tokens, max_positions);
+  if (!start_position_device && (start_position < 0 || (long long)start_position + tokens > max_positions))
+    return fail(FK_ERR_INVALID, "decode positions [%d, %lld) exceed the cache length %d", start_position,
+                (long long)start_position + tokens, max_positions);
   if (!is_float_dtype(cache_dtype) || !is_float_dtype(qk_norm_dtype)) return fail(FK_ERR_DTYPE, "caches and q/k norms must be f32 or bf16");
   if (!key_cache || !value_cache || !o_proj || !q_norm_weight || !k_norm_weight || !update)
     return fail(FK_ERR_INVALID, "attention pointers must be non-NULL");

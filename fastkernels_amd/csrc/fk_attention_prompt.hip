@@ -59,7 +59,7 @@ struct PromptArgs {
 // The start position, or -1 when a device-held one leaves the cache.
 __device__ __forceinline__ int prompt_start(const PromptArgs& a) {
   const int s = a.start_dev ? *a.start_dev : a.start;
-  return s >= 0 && s + a.T <= a.max_pos ? s : -1;
+  return positions_in_cache(s, a.T, a.max_pos) ? s : -1;
 }
 
 template <bool CBF>
@@ -375,7 +375,7 @@ __global__ __launch_bounds__(256) void attn_prompt_merge_kernel(PromptArgs a) {
 // read it).
 __global__ void attn_prompt_advance_kernel(int* start, int T, int max_pos) {
   const int s = *start;
-  if (s >= 0 && s + T <= max_pos) *start = s + T;
+  if (positions_in_cache(s, T, max_pos)) *start = s + T;
 }
 
 struct PromptWs {

@@ -473,6 +473,12 @@ constexpr uint32_t FK_DEVICE_ERR_BARRIER = 1u;
 // step's update is NaN and the position is left where it is.
 constexpr uint32_t FK_DEVICE_ERR_POSITION = 2u;
 
+// Whether positions start .. start + T - 1 lie in a cache of max_pos rows
+// (start + T may pass the range of an int).
+__device__ __forceinline__ bool positions_in_cache(int start, int T, int max_pos) {
+  return start >= 0 && start <= max_pos - T;
+}
+
 __device__ __forceinline__ bool grid_arrive_and_wait(uint32_t* counter, uint32_t target, uint32_t* error,
                                                      uint32_t limit) {
   ticket_add(counter);

@@ -143,6 +143,12 @@ def test_entry_points_reject_bad_arguments_before_launch():
     assert st == _lib.FK_ERR_DTYPE
     st = _err("fk_deltanet_conv", None, 0, None, 0, None, 0, 1, 16, 9, None, None, None)
     assert st == _lib.FK_ERR_UNSUPPORTED
+    # a position whose step would pass the range of an int is past the cache too
+    for fn, dev in (("fk_attention_decode", (None,)), ("fk_attention_prompt", ())):
+        st = _err(fn, *([None, 1] * 2), *([None] * 4), 1, None, None, 1, None, None, 0, 4096, (1 << 31) - 1, *dev,
+                  8, 2048, 16, 2, 256, 64, 1e4, 1, 1e-6, 1e-6, None, None, None, 0, None)
+        assert st == _lib.FK_ERR_INVALID
+        assert b"exceed the cache length" in _lib.load().fk_last_error_detail(), fn
     dts = (ctypes.c_int32 * 10)(*([0] * 10))
     st = _err("fk_deltanet_recurrent_output", *([None] * 10), ctypes.cast(dts, ctypes.c_void_p),
               1, 16, 32, 256, 2048, 1e-6, None, None, None, None, 0, None)

@@ -156,6 +156,27 @@ def test_rows_see_no_later_row():
     assert bool(got[21:].isnan().all())
 
 
+# the single launch, the four launches and the matrix products
+@pytest.mark.parametrize("tokens", [1, 4, 6, 8, 32])
+@pytest.mark.parametrize("position", [-1, 61, 2**31 - 1])
+def test_device_position_past_the_cache(tokens, position):
+    """Also where position + tokens passes the range of an int: NaN, caches
+    untouched, the position left where it is and flagged."""
+
+    x, kc, _, w = _inputs(8, tokens, 2048, 16, 2, 61, torch.bfloat16, torch.float32)
+    names = {"norm_weight": "input_norm_weight", "out_proj_weight": "o_proj_weight"}
+    plan = AttentionStepPlan({names.get(k, k): v for k, v in w.items()}, tokens, max_positions=61, hidden=x)
+    plan.key_cache.copy_(kc)
+    plan.set_position(position)
+    plan.run()
+    torch.cuda.synchronize()
+    assert bool(plan.update.isnan().all()) and int(plan.position) == position
+    assert torch.equal(plan.key_cache, kc)
+    with pytest.raises(_lib.FastKernelsError) as info:
+        plan.check_device()
+    assert info.value.status == _lib.FK_ERR_DEVICE
+
+
 @pytest.mark.parametrize("tokens,start,row", [(8, 1000, 0), (8, 30, 7), (40, 100, 17), (70, 0, 69)])
 def test_infinite_value_of_the_call_stays_infinite(tokens, start, row):
     """One value of one row overflows: the rows that see it get that infinity,
