@@ -1555,7 +1555,10 @@ static size_t attn_ws_layout(int T, int heads, int kvh, int hd, char* base, Attn
   // (hd 256 and G a divisor of 64 are what launch_attn_prompt takes; smaller
   // shapes never need it)
   const bool prompt = T >= kPromptMinTokens && hd == kAttnMaxHeadDim && kvh > 0 && heads % kvh == 0 && heads / kvh <= 8;
-  ws->prompt = take(prompt ? attn_prompt_ws_bytes(T, heads, kvh) : 0);
+  // (its kernels read and write it 16 bytes at a time: the region starts at
+  // the next such boundary where the workspace itself does not lie on one)
+  char* at = take(prompt ? attn_prompt_ws_bytes(T, heads, kvh) + 16 : 0);
+  ws->prompt = reinterpret_cast<char*>(align_up(reinterpret_cast<uintptr_t>(at), 16));
   return off;
 }
 

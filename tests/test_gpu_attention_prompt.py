@@ -156,6 +156,27 @@ def test_rows_see_no_later_row():
     assert bool(got[21:].isnan().all())
 
 
+@pytest.mark.parametrize("tokens", [8, 17])
+def test_decode_workspace_off_the_16_byte_boundary(tokens):
+    """fk_attention_decode asks no alignment of its workspace beyond 8 bytes."""
+
+    x, kc, vc, w = _inputs(9, tokens, 2048, 16, 2, 400, torch.float32, torch.float32)
+    names = {"norm_weight": "input_norm_weight", "out_proj_weight": "o_proj_weight"}
+    plan = AttentionStepPlan({names.get(k, k): v for k, v in w.items()}, tokens, max_positions=400, hidden=x)
+    outs = []
+    for offset in (0, 8):
+        size = plan.workspace.numel()
+        store = torch.zeros(size + 4096, dtype=torch.uint8, device="cuda")
+        plan.workspace = store[offset:offset + size]
+        plan.key_cache.copy_(kc)
+        plan.value_cache.copy_(vc)
+        plan.set_position(300)
+        plan.run()
+        outs.append(plan.update.clone())
+        assert int(store[offset + size:].sum()) == 0
+    assert bool(outs[0].isfinite().all()) and torch.equal(*outs)
+
+
 # the single launch, the four launches and the matrix products
 @pytest.mark.parametrize("tokens", [1, 4, 6, 8, 32])
 @pytest.mark.parametrize("position", [-1, 61, 2**31 - 1])
