@@ -400,18 +400,22 @@ static size_t prompt_ws_layout(int T, int heads, int kvh, char* base, PromptWs* 
   };
   auto floats = [&](size_t n) { return reinterpret_cast<float*>(take(n * 4)); };
   const size_t q = (size_t)T * heads * kPromptHd, kv = (size_t)T * kvh * kPromptHd;
-  const size_t nc = (size_t)prompt_max_chunks(T, heads, kvh);
+  // rows of chunk partials: at most kPromptWgs * kPromptRows from two chunks on,
+  // whatever T (as a bound that never falls, so that a size that is enough for
+  // T rows is enough for fewer)
+  const size_t th = (size_t)T * heads, most = (size_t)kPromptWgs * kPromptRows;
+  const size_t parts = th > most ? th : th * kPromptMaxChunks < most ? th * kPromptMaxChunks : most;
   ws->qg = floats(2 * q);
   ws->k = floats(kv);
   ws->v = floats(kv);
   ws->q_rot = floats(q);
   ws->k_rot = floats(kv);
   ws->v_bad = reinterpret_cast<int*>(take((size_t)T * kvh * 4));
-  ws->stat = floats((size_t)T * heads * nc * 2);
-  ws->acc = floats(q * nc);
+  ws->stat = floats(parts * 2);
+  ws->acc = floats(parts * kPromptHd);
   ws->planes = reinterpret_cast<uint16_t*>(take(q * 6));
   ws->part_bytes = token_part_bytes(T);
-  ws->part = reinterpret_cast<float*>(take(ws->part_bytes));
+  ws->part = reinterpret_cast<float*>(take(token_part_reserve(T)));
   return off;
 }
 

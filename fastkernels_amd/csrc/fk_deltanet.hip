@@ -61,7 +61,7 @@ static size_t dn_ws_layout(int T, int Hv, int D, char* base, DnWs* ws) {
   ws->planes = reinterpret_cast<uint16_t*>(take((size_t)T * Hv * D * 6));
   ws->normed = reinterpret_cast<float*>(ws->planes);
   ws->part_bytes = token_part_bytes(T);
-  ws->part = reinterpret_cast<float*>(take(ws->part_bytes));
+  ws->part = reinterpret_cast<float*>(take(token_part_reserve(T)));
   return off;
 }
 

@@ -49,12 +49,15 @@ int launch_plane_gemm(const uint16_t* planes, const void* w, int R, int T, int K
                       int residual_dt, float* out, float* residual_out, float* part, size_t part_bytes,
                       hipStream_t s);
 
-// Bytes for launch_plane_gemm's partial sums of 2,048 output rows: up to 8
-// splits of K, fewer as the tokens fill the chip by themselves.
+// Bytes that launch_plane_gemm's partial sums of 2,048 output rows may take: up
+// to 8 splits of K, fewer as the tokens fill the chip by themselves.  A
+// workspace holds token_part_reserve of them, the most that T tokens or fewer
+// take: a size that is enough for a number of tokens is enough for fewer.
 inline size_t token_part_bytes(int T) {
   const size_t splits = T >= 1024 ? 1 : T <= 128 ? 8 : (size_t)(1024 / T);
   return splits > 1 ? splits * (size_t)T * 2048 * 4 : 0;
 }
+inline size_t token_part_reserve(int T) { return token_part_bytes(T < 128 ? T : 128); }
 
 // Gated attention over T rows of one sequence as a prompt
 // (fk_attention_prompt.hip), at the shapes attn_prompt_ok takes; `err` is the

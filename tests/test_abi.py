@@ -116,6 +116,34 @@ def test_workspace_sizes_are_monotone():
     assert lib.fk_deltanet_workspace_bytes(8, 32, 128) >= 2 * 8 * 32 * 128 * 4
 
 
+@pytest.mark.parametrize("heads,kv_heads,value_heads", [(16, 2, 32), (8, 4, 4), (4, 4, 5), (1, 1, 2)])
+def test_workspace_sizes_never_fall(heads, kv_heads, value_heads):
+    """A workspace sized for a number of tokens is enough for fewer: a caller
+    that sizes one for its longest chunk runs the shorter last one on it."""
+
+    lib = _lib.load()
+    sizes = {
+        "deltanet": [lib.fk_deltanet_workspace_bytes(t, value_heads, 128) for t in range(1, 1300)],
+        "deltanet step": [lib.fk_deltanet_step_workspace_bytes(t, 1, value_heads, 128) for t in range(1, 65)],
+        "attention prompt": [lib.fk_attention_prompt_workspace_bytes(t, 2048, heads, kv_heads, 256, 1, 1)
+                             for t in range(1, 2500)],
+        "attention": [lib.fk_attention_workspace_bytes(t, heads, kv_heads, 256) for t in range(8, 33)],
+    }
+    for name, s in sizes.items():
+        assert 0 < s[0] and all(a <= b for a, b in zip(s, s[1:])), name
+
+
+@pytest.mark.parametrize("heads,kv_heads", [(16, 2), (8, 4), (16, 16), (5, 5), (8, 1), (1, 1)])
+def test_prompt_chunk_partials_fit(heads, kv_heads):
+    """The bound on the prompt's chunk partials covers what every T takes: 512
+    workgroups of 64 query rows over kv heads and row blocks, at most 64 chunks."""
+
+    for t in range(1, 3000):
+        chunks = min(64, max(1, 512 // (-(-t * (heads // kv_heads) // 64) * kv_heads)))
+        th = t * heads
+        assert th * chunks <= max(th, min(th * 64, 512 * 64)), t
+
+
 def _err(fn: str, *args) -> int:
     lib = _lib.load()
     return getattr(lib, fn)(*args)
