@@ -969,6 +969,11 @@ def hip_qwen36_batched_attention_project(
 
 
 _MAX_ATTN_ROWS = 32  # rows per fk_attention_decode call (fk_attention.hip kAttnMaxTokens)
+# Rows per fk_attention_prompt call.  Its workspace, which stays with the stream, grows with them (124 MB here at the
+# model's shape, about 90 KB for each row more), and past it the causal triangle leaves workgroups idle: 4,096 rows take 4.5 ms
+# in calls of 1,024, 6.7 in calls of 2,048 and 6.5 in one.  Rows of the calls before are read from the cache, so from a
+# bf16 one as it rounds them; a call's own enter unrounded.
+_MAX_PROMPT_ROWS = 1024
 
 
 def _attention(hidden, key_cache, value_cache, norm_weight, q_proj_weight, k_proj_weight, v_proj_weight,
@@ -1017,22 +1022,25 @@ def _attention(hidden, key_cache, value_cache, norm_weight, q_proj_weight, k_pro
     out = torch.empty_like(update) if residual else None
     lib = _lib.load()
     if tokens > _MAX_ATTN_ROWS:
-        # a prompt: one call for any number of rows, at the shapes it takes
+        # a prompt: calls of up to _MAX_PROMPT_ROWS rows, at the shapes they take
         nbytes = lib.fk_attention_prompt_workspace_bytes(
-            tokens, hidden_size, attention_heads, kv_heads, head_dim, _fcode(wq, "projection weights"),
-            _fcode(nw, "norm_weight"))
+            min(tokens, _MAX_PROMPT_ROWS), hidden_size, attention_heads, kv_heads, head_dim,
+            _fcode(wq, "projection weights"), _fcode(nw, "norm_weight"))
         if nbytes:
             ws = _workspace("attention_prompt", dev, nbytes)
-            _lib.call(
-                "fk_attention_prompt",
-                x.data_ptr(), _fcode(x, "hidden"), nw.data_ptr(), _fcode(nw, "norm_weight"),
-                wq.data_ptr(), wk.data_ptr(), wv.data_ptr(), wo.data_ptr(), _fcode(wq, "projection weights"),
-                qn.data_ptr(), kn.data_ptr(), _fcode(qn, "q_norm_weight"),
-                kc.data_ptr(), vc.data_ptr(), _fcode(kc, "key_cache"), kc.shape[0], int(start_position),
-                tokens, hidden_size, attention_heads, kv_heads, head_dim, int(rope_dim), float(rope_theta),
-                1 if rope_interleaved else 0, float(eps), float(qk_norm_eps),
-                update.data_ptr(), _ptr(out), ws.data_ptr(), ws.numel(), _stream(dev),
-            )
+            for s in range(0, tokens, _MAX_PROMPT_ROWS):
+                e = min(tokens, s + _MAX_PROMPT_ROWS)
+                _lib.call(
+                    "fk_attention_prompt",
+                    x[s:e].data_ptr(), _fcode(x, "hidden"), nw.data_ptr(), _fcode(nw, "norm_weight"),
+                    wq.data_ptr(), wk.data_ptr(), wv.data_ptr(), wo.data_ptr(), _fcode(wq, "projection weights"),
+                    qn.data_ptr(), kn.data_ptr(), _fcode(qn, "q_norm_weight"),
+                    kc.data_ptr(), vc.data_ptr(), _fcode(kc, "key_cache"), kc.shape[0], int(start_position) + s,
+                    e - s, hidden_size, attention_heads, kv_heads, head_dim, int(rope_dim), float(rope_theta),
+                    1 if rope_interleaved else 0, float(eps), float(qk_norm_eps),
+                    update[s:e].data_ptr(), _ptr(out[s:e] if out is not None else None), ws.data_ptr(), ws.numel(),
+                    _stream(dev),
+                )
             return update, out, kc, vc
     # fk_attention_decode takes at most _MAX_ATTN_ROWS rows per call (their new
     # keys sit in LDS on its general path); longer batches go through in consecutive calls: each call

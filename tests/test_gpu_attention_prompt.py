@@ -97,6 +97,49 @@ def _error(seed, tokens, start, hidden, heads, kvh, cache_dtype, q_norm=1.0):
     return float((got.double() - ref).norm() / ref.norm())
 
 
+def test_long_prompt_in_calls_of_bounded_size():
+    """2,100 rows: three calls on one workspace that no longer prompt grows, as
+    one call of the C entry (a single chunk of positions per workgroup) gives."""
+
+    tokens, start = 2100, 5
+    x, kc, vc, w = _inputs(12, tokens, 512, 16, 2, start + tokens, torch.float32, torch.float32)
+    hip._workspaces.clear()
+    update, k, v = hip.hip_qwen36_batched_attention_decode(x, kc, vc, *w.values(), start_position=start)
+    lib = _lib.load()
+    kept = [t.numel() for (kind, _, _), t in hip._workspaces.items() if kind == "attention_prompt"]
+    assert kept == [lib.fk_attention_prompt_workspace_bytes(1024, 512, 16, 2, 256, 1, 1)]
+    ref, rk, _ = _reference(x, kc, vc, w, start, 16, 2, 64, 1e4, True)
+    tol = 2e-6 + tokens * 2.0 ** -24 * 0.5  # (as test_prompt_rows)
+    assert float((update.double() - ref).norm() / ref.norm()) < tol
+    assert torch.allclose(k[start:].double(), rk, rtol=tokens * 2.0 ** -23, atol=tokens * 2.0 ** -23)
+
+    one, k2, v2 = torch.empty_like(update), kc.clone(), vc.clone()
+    n = lib.fk_attention_prompt_workspace_bytes(tokens, 512, 16, 2, 256, 1, 1)
+    ws = torch.zeros(n, dtype=torch.uint8, device="cuda")
+    p = {name: t.data_ptr() for name, t in w.items()}
+    _lib.call("fk_attention_prompt", x.data_ptr(), 0, p["norm_weight"], 1, p["q_proj_weight"], p["k_proj_weight"],
+              p["v_proj_weight"], p["out_proj_weight"], 1, p["q_norm_weight"], p["k_norm_weight"], 1, k2.data_ptr(),
+              v2.data_ptr(), 0, start + tokens, start, tokens, 512, 16, 2, 256, 64, 1e4, 1, 1e-6, 1e-6, one.data_ptr(),
+              None, ws.data_ptr(), n, torch.cuda.current_stream().cuda_stream)
+    assert float((one.double() - ref).norm() / ref.norm()) < tol
+    # (sums over K in the same steps whatever the tile: the last bits of the larger tiles aside)
+    assert torch.allclose(k2, k, rtol=1e-4, atol=1e-5) and torch.allclose(v2, v, rtol=1e-4, atol=1e-5)
+
+
+@pytest.mark.parametrize("tokens", [700, 1030])
+def test_long_prompt_residual(tokens):
+    """The layer's hidden states, written by the larger tiles of the output
+    projection (700 rows: K unsplit; a second call of 6)."""
+
+    x, kc, vc, w = _inputs(13, tokens, 2048, 16, 2, tokens, torch.bfloat16, torch.float32)
+    gen = torch.Generator().manual_seed(14)
+    moe = [_randn(gen, s, 0.02) for s in ((2048,), (16, 2048), (16, 128, 2048), (16, 2048, 64), (128, 2048), (2048, 64), (2048,))]
+    _, hidden, update, *_ = hip.hip_qwen36_batched_attention_moe_layer_decode(x, kc, vc, *w.values(), *moe, top_k=2)
+    ref, _, _ = _reference(x, kc, vc, w, 0, 16, 2, 64, 1e4, True)
+    assert float((update.double() - ref).norm() / ref.norm()) < 2e-6 + tokens * 2.0 ** -24 * 0.5
+    assert torch.equal(hidden, x.float() + update)
+
+
 # A score is a sum of 256 products, whose roundings all reach the output.  In
 # short chains added in pairs, as the dot products of few rows are (4 products
 # and 6 levels), the variance is about 8 to 12 squared roundings of the score;
