@@ -36,6 +36,7 @@
 #include "fk_common.h"
 #include "fk_host.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace fk {
@@ -482,9 +483,18 @@ struct AttnProjArgs {
 };
 constexpr int kAttnProjRows = 16;
 // From this many tokens fk_attention_project runs on the matrix cores
-// (launch_norm_gemm: 24.3 us at 3 to 32 tokens, the model's 9,216 rows, 55-60
-// at 256, where this kernel takes 22.6 us at 8, 28.6 at 12 and 406 at 256).
-constexpr int kAttnGemmMinTokens = 10;
+// (launch_norm_gemm), whose time at 1 to 32 tokens follows K and hardly the
+// rows, where this kernel's follows the tokens and its workgroups per CU.  Both
+// sides, us, this kernel / the matrix cores: 9,216 rows (the model's), K 2048,
+// fp32 tokens 21.8 at 9, 23.5 at 10, 24.8 at 11, 26.5 at 12 / 24.4 to 25.4
+// (bf16 21.5, 23.0, 24.6, 26.0 / 25.2 to 25.9), K 1024 16.4 at 10 / 14.3; 5,120
+// rows, K 2048 24.0 at 16, 26.4 at 18 / 24.2; 6,144 rows, K 1024 13.2 at 11,
+// 14.2 at 12 / 14.3; 3,072 rows, K 1024 13.3 at 16 / 14.1; 1,024 rows, K 2048
+// 14.4 at 12, 20.5 at 20, 24.3 at 24 / 23.5; 1,536 rows, K 512 7.9 at 10, 8.8 at
+// 12 / 8.2; 768 rows, K 64 8.3 at 10 / 4.6.
+static int attn_gemm_min_tokens(int R, int K) {
+  return std::max(10, R <= 4096 ? 7 + K / 120 : R <= 7168 ? 7 + K / 200 : 4 + K / 256);
+}
 
 template <bool BFW, bool BFX>
 __global__ __launch_bounds__(256) void attn_proj_kernel(AttnProjArgs a) {
@@ -1654,7 +1664,7 @@ int fk_attention_project(const void* hidden, int hidden_dtype, const void* norm_
   const void* const w[4] = {q_proj, k_proj, v_proj, nullptr};
   const int rows[4] = {q_rows, kv_rows, kv_rows, 0};
   float* const out[4] = {q_out, k_out, v_out, nullptr};
-  if (tokens >= kAttnGemmMinTokens && norm_gemm_ok(rows, hidden_size, weight_dtype, norm_dtype))
+  if (tokens >= attn_gemm_min_tokens(q_rows + 2 * kv_rows, hidden_size) && norm_gemm_ok(rows, hidden_size, weight_dtype, norm_dtype))
     return launch_norm_gemm(hidden, hidden_dtype, norm_weight, w, rows, out, tokens, hidden_size, eps, norm_offset,
                             as_stream(stream));
   if (hidden_size <= 2048 && q_rows % 4 == 0 && kv_rows % 4 == 0) {

@@ -13,7 +13,7 @@
 //   deltanet_project_kernel   grid ceil(R/16): 16 rows of the concatenated
 //                             [qkv | z | a | b] weight space per workgroup,
 //                             streamed once and applied to every token; batches
-//                             of kGemmMinTokens or more at the shapes norm_gemm_ok
+//                             of proj_gemm_min_tokens or more at the shapes norm_gemm_ok
 //                             takes run token_gemm_kernel (fk_gemm.hip) instead.
 //   deltanet_conv_kernel      a thread per channel and block of 8 rows, sliding
 //                             window in registers.
@@ -89,9 +89,21 @@ struct ProjArgs {
 
 constexpr int kProjMaxFusedTokens = 64;
 // From this many tokens the projections run on the matrix cores
-// (launch_norm_gemm): 25-26 us at 3 to 32 tokens where this kernel takes 24.0
-// us at 2, 29.8 at 4 and 41.6 at 8 (the model's 12,352 rows).
-constexpr int kGemmMinTokens = 4;
+// (launch_norm_gemm), whose time at 1 to 32 tokens follows K and hardly the
+// rows, where this kernel's rises with the tokens, and more so once its
+// workgroups of 16 rows are more than the CUs hold at once (2 each, of its
+// wide form for K above 2048 one).  Both sides, us, this kernel / the matrix
+// cores: 12,352 rows (the model's), K 2048 24.3 at 3, 26.6 (bf16 tokens 27.8) at
+// 4, 38.0 at 8 / 25.3 to 26.1, K 1024 16.1 at 3, 18.1 at 4 / 15, K 512 13.5 at 4
+// / 9.3; 8,256 rows, K 2048 20.8 at 3, 24.9 at 4, 27.5 at 5 / 24.5; 6,176 rows,
+// K 2048 19.2 at 7, 22.4 at 10 / 24.1, K 4096 47.6 at 5 / 44.9; 3,104 rows, K
+// 4096 38.4 at 10, 44.7 at 12 / 44; 1,056 rows, K 2048 19.8 at 9, 22.6 at 11 /
+// 23.6, K 1024 11.3 at 7, 12.1 at 8 / 12.5; 1,568 rows, K 512 7.3 at 4, 8.6 at 6
+// / 8.4; 544 rows, K 64 7.9 at 4 / 4.5.
+static int proj_gemm_min_tokens(int R, int K) {
+  if (K < 512 || R > (K > 2048 ? 4096 : 8192)) return 4;
+  return K < 1024 ? 6 : K < 2048 ? 9 : 12;
+}
 // From this many tokens the recurrence runs as the scan and the output
 // projection on the matrix cores, two to three more launches: the operator
 // takes 28 us from 3 to 32 tokens where the two kernels before took 24.5 us at
@@ -2021,9 +2033,9 @@ __global__ __launch_bounds__(512) void deltanet_step_kernel(StepArgs a) {
 // Host launchers
 // ---------------------------------------------------------------------------
 static int launch_project(const ProjArgs& pa, int weight_dtype, int hidden_dtype, hipStream_t s) {
-  if (!pa.conv_out && pa.T >= kGemmMinTokens && norm_gemm_ok(pa.rows, pa.H, weight_dtype, pa.nw_dt))
-    return launch_norm_gemm(pa.x, hidden_dtype, pa.nw, pa.w, pa.rows, pa.out, pa.T, pa.H, pa.eps, pa.off, s);
   const int R = pa.rows[0] + pa.rows[1] + pa.rows[2] + pa.rows[3];
+  if (!pa.conv_out && pa.T >= proj_gemm_min_tokens(R, pa.H) && norm_gemm_ok(pa.rows, pa.H, weight_dtype, pa.nw_dt))
+    return launch_norm_gemm(pa.x, hidden_dtype, pa.nw, pa.w, pa.rows, pa.out, pa.T, pa.H, pa.eps, pa.off, s);
   const int grid = (R + kProjRows - 1) / kProjRows;
   const bool bfw = weight_dtype == FK_DTYPE_BF16, bfx = hidden_dtype == FK_DTYPE_BF16, wide = pa.H > 2048;
 #define FK_PROJ(BW, BX)                                                                                   \
@@ -2489,7 +2501,8 @@ int fk_deltanet_step(const void* hidden, const void* input_norm_weight, const vo
   pa.KS = kernel_size;
   pa.conv_out = ws.mixed;
   pa.next_state = next_conv_state;
-  if (tokens >= kGemmMinTokens && norm_gemm_ok(pa.rows, hidden_size, dtypes[2], dtypes[1])) {
+  const int R = conv_dim + (head_dim + 2) * value_heads;
+  if (tokens >= proj_gemm_min_tokens(R, hidden_size) && norm_gemm_ok(pa.rows, hidden_size, dtypes[2], dtypes[1])) {
     pa.out[0] = ws.raw;
     st = launch_norm_gemm(hidden, dtypes[0], input_norm_weight, pa.w, pa.rows, pa.out, tokens, hidden_size, eps, 1.0f, s);
     if (st) return st;

@@ -42,6 +42,11 @@ def _check(outs, x, norm, weights, eps=1e-6):
     (129, 2048, (8192, 4096, 32), torch.float32),
     (257, 1024, (8192, 4096, 32), torch.float32),
     (400, 4096, (8192, 4096, 32), torch.float32),
+    # either side of the rule's lines for few rows
+    (11, 2048, (512, 256, 16), torch.float32),
+    (12, 2048, (512, 256, 16), torch.bfloat16),
+    (8, 1024, (512, 256, 16), torch.float32),
+    (9, 1024, (512, 256, 16), torch.float32),
 ])
 def test_deltanet_projection_batches(tokens, hidden, rows, x_dtype):
     gen = torch.Generator().manual_seed(tokens)
@@ -54,7 +59,7 @@ def test_deltanet_projection_batches(tokens, hidden, rows, x_dtype):
     assert all(torch.equal(a, b) for a, b in zip(outs, again))
 
 
-@pytest.mark.parametrize("tokens", [10, 40, 200])
+@pytest.mark.parametrize("tokens", [10, 11, 12, 40, 200])
 def test_attention_projection_batches(tokens):
     gen = torch.Generator().manual_seed(tokens)
     x, norm = _randn(gen, (tokens, 2048), 1.0, torch.float32), _randn(gen, (2048,), 0.1)
