@@ -2932,6 +2932,20 @@ static int launch_router_tagged_t(const RouterArgs& ra_in, hipStream_t stream) {
   return check_launch("moe_router_tagged_kernel");
 }
 
+// Calls past the tagged router that take the matrix cores: the products' time
+// at up to 112 tokens follows the hidden size (0.7 us per 64), the grid-barrier
+// kernel's the tokens times the experts (and more slowly where its wide form
+// reads more than 2,048 values a row).  Both sides, us, that kernel / the
+// matrix cores: 512 experts, H 512 20.6 at 6, 22.7 at 8, 25.0 at 12 / 23; H 1024
+// 26.6 at 12, 28.9 at 16 / 28; H 2048 34.1 at 16, 39.7 at 32 / 36; H 4096 51 at
+// 32, 64 at 48 / 55; 1,024 experts, H 2048 35 at 12, 40 at 16 / 39, H 4096 52 at
+// 16, 63 at 24 / 58; 256 experts, H 3072 35 at 32, 40 at 48 / 38; 64 experts, H
+// 4096 42 at 64, 46 at 100 / 47 to 48.
+static bool router_gemm_pays(const RouterArgs& ra) {
+  const long long work = (long long)ra.T * ra.E;
+  return ra.T >= 112 || work > (ra.H > 2048 ? 4ll : 8ll) * ra.H;
+}
+
 static int launch_router(const RouterArgs& ra, int router_dt, int hidden_dt, hipStream_t stream) {
   const bool bfw = router_dt == FK_DTYPE_BF16, bfx = hidden_dt == FK_DTYPE_BF16;
   if (tagged_router_eligible(ra)) {
@@ -2949,7 +2963,7 @@ static int launch_router(const RouterArgs& ra, int router_dt, int hidden_dt, hip
   // shape: 179 -> 43 us against the grid-barrier kernel below, whose VALU
   // logits take ~0.3 us a token and whose last workgroup builds the tables).
   const int rows[4] = {ra.E, 0, 0, 0};
-  if (norm_gemm_ok(rows, ra.H, router_dt, ra.nw_dt)) {
+  if (router_gemm_pays(ra) && norm_gemm_ok(rows, ra.H, router_dt, ra.nw_dt)) {
     const void* const w[4] = {ra.W, nullptr, nullptr, nullptr};
     float* const out[4] = {ra.logits, nullptr, nullptr, nullptr};
     st = launch_norm_gemm(ra.x, hidden_dt, ra.nw, w, rows, out, ra.T, ra.H, ra.eps, ra.off, stream);

@@ -113,6 +113,13 @@ def test_routing_tables(pairs, experts):
     (300, 512, 48, 3, True, torch.bfloat16),
     (512, 1024, 1024, 8, True, torch.float32),
     (20, 64, 272, 8, False, torch.float32),
+    # more than 256 experts or 2,048 values: either side of the line between the kernels
+    (1, 512, 1024, 8, True, torch.float32),
+    (4, 512, 1024, 8, False, torch.bfloat16),
+    (5, 512, 1024, 8, False, torch.bfloat16),
+    (64, 4096, 256, 8, False, torch.float32),
+    (65, 4096, 256, 8, True, torch.float32),
+    (112, 3072, 16, 4, True, torch.float32),
 ])
 def test_router_batches(tokens, hidden, experts, top_k, bias, dtype):
     from oracle import qwen36 as oracle
