@@ -1086,7 +1086,7 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(ExpertArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Batched expert stage (bf16 weights; T >= 44 bf16 or 84 fp32 tokens):
+// Batched expert stage (bf16 weights; T >= 44 bf16 tokens, or fp32 ones as f32_mfma_pays has it):
 // MFMA grouped GEMM over the routing tables.
 //
 // Weight rows are loaded row-contiguously (a wavefront's K range of a row
@@ -1318,10 +1318,22 @@ constexpr int kGtAhead = 2;   // weight steps in flight (two workgroups on a CU;
 // 311, 390 / 336.
 constexpr int kGtWidePairs = 12;
 // fp32 hidden states take the MFMA kernels from this many tokens (expert
-// stage, GEMV / MFMA: 238 / 259 us at 64, 298 / 280 at 96, 359 / 298 at 128,
-// 562 / 310 at 256, 1035 / 352 at 512: the GEMV kernels apply the rows once
-// per pair).
+// stage of the model's shapes, GEMV / MFMA: 238 / 259 us at 64, 298 / 280 at 96,
+// 359 / 298 at 128, 562 / 310 at 256, 1035 / 352 at 512: the GEMV kernels apply
+// the rows once per pair), with a shared expert, whose GEMV is a row of all
+// tokens, at any pairs per routed expert (0.33 pairs, 84 tokens: 182 / 107).
+// Routed experts alone need pairs to pay for the split tokens: 3 per expert of
+// H x I = 2^20 and in proportion for smaller ones (GEMV / MFMA: 256 experts of
+// 2048 x 512 234 / 258 at 2 pairs, 270 / 281 at 2.5, 298 / 285 at 3; 64 experts
+// 87 / 92 at 3, 100 / 95 at 4; 128 of 1024 x 512 74 / 77 at 1.75, 79 / 80 at 2;
+// 1,024 of 2048 x 256 225 / 254 at 0.5, 387 / 382 at 1; 1,024 of 1024 x 256 123 /
+// 128 at 0.5, 168 / 163 at 0.75; 512 of 512 x 256 35 / 40 at 0.31, 48 / 49 at
+// 0.5, 55 / 53 at 0.62).
 constexpr int kMfmaMinTokensF32 = 84;
+static bool f32_mfma_pays(const ExpertArgs& ea) {
+  if (ea.T < kMfmaMinTokensF32) return false;
+  return ea.has_shared || ((long long)ea.T * ea.K << 20) >= 3ll * ea.E * ea.H * ea.I;
+}
 
 template <int BM, int NP>
 __global__ __launch_bounds__(512, 4) void moe_gateup_tile_kernel(ExpertArgs a, int items) {
@@ -3059,7 +3071,7 @@ static int launch_experts(const ExpertArgs& ea, int expert_dt, hipStream_t strea
   const int max_active = ea.T * ea.K < ea.E ? ea.T * ea.K : ea.E;
   const int slots = max_active + (ea.has_shared ? 1 : 0);
   int st = FK_OK;
-  if (ea.T >= (bfx ? kMfmaMinTokens : kMfmaMinTokensF32) && bfw && mfma_expert_shapes_ok(ea.H, ea.I)) {
+  if ((bfx ? ea.T >= kMfmaMinTokens : f32_mfma_pays(ea)) && bfw && mfma_expert_shapes_ok(ea.H, ea.I)) {
     st = launch_experts_mfma(ea, bfx, slots, stream);
     if (st) return st;
   } else {

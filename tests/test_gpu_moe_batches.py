@@ -45,6 +45,9 @@ def _reference(x, ids, w, gu, dn, sgu=None, sdn=None, sg=None):
     (150, 1024, 256, 4, 3, True),    # 112 pairs an expert: further tiles
     (300, 1024, 512, 3, 2, False),
     (512, 2048, 256, 256, 8, True),
+    # routed experts alone: fewer pairs than the fp32 line (3 an expert of 2048 x 512) and at it
+    (95, 2048, 512, 64, 2, False),
+    (96, 2048, 512, 64, 2, False),
 ])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_expert_batches(tokens, hidden, inter, experts, top_k, shared, dtype):
