@@ -132,8 +132,8 @@ __device__ __forceinline__ int wave_incl_scan(int v, int lane) {
 // Deterministic, parallel stable counting sort of the P pairs by expert.
 // Wave w owns the contiguous pair segment [w*seg, (w+1)*seg); it walks it in
 // chunks of 64 (one pair per lane), ranks each pair among equal experts of
-// the chunk by scanning the 64 ids through readlane broadcasts, and keeps
-// running per-expert counts of its segment in s_wcnt[w][e].  A pair's
+// the chunk by a ballot per id bit (fewer pairs than bits: a readlane per
+// pair), and keeps running per-expert counts of its segment in s_wcnt[w][e].  A pair's
 // permuted position is offsets[e] + (pairs of e in earlier segments) +
 // (its rank inside its own segment), which preserves (token, slot) order.
 // It also writes one record per active expert (ws.slots: id, first position,
@@ -156,12 +156,18 @@ __device__ void build_routing_tables(const int* s_ids, int P, int E, int K, MoeW
     const int j = c0 + lane;
     const bool valid = j < j1;
     const int e = valid ? s_ids[j] : 0;
-    // the chunk's lanes with this lane's expert: one ballot per id bit (a
-    // readlane per lane took 64 rounds a chunk: 50 us for 2,664 pairs)
-    uint64_t same = __ballot(valid);
-    for (int q = 0; q < ebits; ++q) {
-      const uint64_t bit = __ballot((e >> q) & 1);
-      same &= (e >> q) & 1 ? bit : ~bit;
+    // the chunk's lanes with this lane's expert (a readlane for each of 64
+    // lanes took 50 us for 2,664 pairs)
+    uint64_t same = 0;
+    const int n = min(kWave, j1 - c0);
+    if (n <= ebits) {
+      for (int src = 0; src < n; ++src) same |= (uint64_t)(__builtin_amdgcn_readlane(e, src) == e) << src;
+    } else {
+      same = __ballot(valid);
+      for (int q = 0; q < ebits; ++q) {
+        const uint64_t bit = __ballot((e >> q) & 1);
+        same &= (e >> q) & 1 ? bit : ~bit;
+      }
     }
     const int below = __popcll(same & ((1ull << lane) - 1ull)), total = __popcll(same);
     int before = 0;
@@ -750,12 +756,15 @@ struct AlignArgs {
   int32_t* inverse_out;
 };
 
-constexpr int kAlignWaves = 16;  // (four wavefronts and a readlane per pair: 50 us at 2,664 pairs; now 9)
-__global__ __launch_bounds__(64 * kAlignWaves) void moe_align_kernel(AlignArgs a) {
-  constexpr int NTH = 64 * kAlignWaves;
+// NWV wavefronts: 4 up to kAlignFewPairs pairs, else 16 (us, 4 / 16: 8 pairs of
+// 256 experts 4.4 / 5.4, 32 4.7 / 5.7; 2,664 pairs 9 with 16).
+constexpr int kAlignFewPairs = 128;
+template <int NWV>
+__global__ __launch_bounds__(64 * NWV) void moe_align_kernel(AlignArgs a) {
+  constexpr int NTH = 64 * NWV;
   __shared__ int s_ids[kMaxPairs];
   __shared__ int s_rank[kMaxPairs];
-  __shared__ int s_wcnt[kAlignWaves * kMaxExperts];
+  __shared__ int s_wcnt[NWV * kMaxExperts];
   __shared__ int s_cnt[kMaxExperts];
   __shared__ int s_off[kMaxExperts];
   __shared__ int s_aidx[kMaxExperts];
@@ -773,7 +782,7 @@ __global__ __launch_bounds__(64 * kAlignWaves) void moe_align_kernel(AlignArgs a
     a.ws.wts[j] = a.w ? load_scalar(a.w, a.w_dt, j) : 0.f;
   }
   __syncthreads();
-  build_routing_tables<kAlignWaves>(s_ids, P, a.E, a.K, a.ws, s_cnt, s_off, s_rank, s_wcnt, s_aidx);
+  build_routing_tables<NWV>(s_ids, P, a.E, a.K, a.ws, s_cnt, s_off, s_rank, s_wcnt, s_aidx);
   __syncthreads();
   // Optional copies of the tables for callers that inspect them.
   for (int e = threadIdx.x; e < a.E; e += NTH) {
@@ -2944,6 +2953,12 @@ static int launch_router_tagged_t(const RouterArgs& ra_in, hipStream_t stream) {
   return check_launch("moe_router_tagged_kernel");
 }
 
+static int launch_align(const AlignArgs& aa, hipStream_t stream) {
+  if (aa.T * aa.K <= kAlignFewPairs) hipLaunchKernelGGL(moe_align_kernel<4>, dim3(1), dim3(256), 0, stream, aa);
+  else hipLaunchKernelGGL(moe_align_kernel<16>, dim3(1), dim3(1024), 0, stream, aa);
+  return check_launch("moe_align_kernel");
+}
+
 // Calls past the tagged router that take the matrix cores: the products' time
 // at up to 112 tokens follows the hidden size (0.7 us per 64), the grid-barrier
 // kernel's the tokens times the experts (and more slowly where its wide form
@@ -2990,8 +3005,7 @@ static int launch_router(const RouterArgs& ra, int router_dt, int hidden_dt, hip
     aa.K = ra.K;
     aa.E = ra.E;
     aa.ws = ra.ws;
-    hipLaunchKernelGGL(moe_align_kernel, dim3(1), dim3(64 * kAlignWaves), 0, stream, aa);
-    return check_launch("moe_align_kernel");
+    return launch_align(aa, stream);
   }
   FK_DISPATCH_BOOL(bfw, BW, FK_DISPATCH_BOOL(bfx, BX, {
     if (wide) st = many ? launch_router_t<BW, BX, 8, 16>(ra, stream) : launch_router_t<BW, BX, 8, 4>(ra, stream);
@@ -3282,8 +3296,7 @@ int fk_moe_align(const void* topk_ids, int ids_dtype, const void* topk_weights, 
   aa.offsets_out = offsets_out;
   aa.perm_out = perm_out;
   aa.inverse_out = inverse_out;
-  hipLaunchKernelGGL(moe_align_kernel, dim3(1), dim3(64 * kAlignWaves), 0, as_stream(stream), aa);
-  return check_launch("moe_align_kernel");
+  return launch_align(aa, as_stream(stream));
 }
 
 int fk_moe_experts(const void* hidden, int hidden_dtype, const void* gate_up, const void* down, int expert_dtype,

@@ -98,7 +98,7 @@ def test_values_past_the_bf16_range():
     assert float((out.double() - ref).norm() / ref.norm()) < 1e-6
 
 
-@pytest.mark.parametrize("pairs,experts", [(1, 1), (63, 3), (64, 256), (65, 2), (1023, 7), (1030, 1024), (4096, 256), (4096, 1)])
+@pytest.mark.parametrize("pairs,experts", [(1, 1), (63, 3), (64, 256), (65, 2), (128, 256), (136, 1000), (40, 8), (1023, 7), (1030, 1024), (4096, 256), (4096, 1)])
 def test_routing_tables(pairs, experts):
     from oracle import qwen36 as oracle
 
