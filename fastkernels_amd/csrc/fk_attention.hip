@@ -14,8 +14,8 @@
 //   update = (o * sigmoid(gate)) Wo^T;  hidden_out = x + update
 //
 // Kernels: T <= 4 at the shapes attn_step_chunks accepts (the model's) run
-// as one launch, attn_step_kernel (below); 8 rows or more at the shapes
-// attn_prompt_ok accepts as matrix products (fk_attention_prompt.hip); other
+// as one launch, attn_step_kernel (below); prompt_min_tokens rows or more at
+// the shapes attn_prompt_ok accepts as matrix products (fk_attention_prompt.hip); other
 // steps as four launches:
 //   attn_proj_kernel  RMSNorm folded into a GEMV over [Wq | Wk | Wv] (9216
 //                     rows at the model shape); H > 2048 takes the shared
@@ -45,9 +45,26 @@ constexpr int kAttnMaxHeadDim = 256;
 constexpr int kAttnMaxTokens = 32;  // new keys of the step are kept in LDS (T * hd floats)
 constexpr int kAttnOutRows = 4;  // Wo rows per out-projection workgroup (1 per wavefront)
 // From this many rows launch_attn_prompt's kernels replace the four launches
-// below (58 against 68 us at 5 rows behind 1,000 positions, 65 / 61 at 8
-// behind 100, 126 / 73 at 16, 195 / 71 at 32).
+// below, whose time follows the rows, the heads and the kv heads (with few of
+// them the products are as many launches with less to do).  Both sides, us,
+// four launches / matrix products, behind 10 and 1,000 positions: 16 heads of 2
+// kv heads, 8 rows 57 / 58 and 77 / 73, 16 rows 94 / 59 and 132 / 75; 8 of 8,
+// hidden 512, 8 rows 35 / 35 and 69 / 45; 12 of 3 63 / 59 behind 1,000; 8 of 2
+// 36 / 42 and 45 / 49, 10 rows level; 8 of 1, hidden 512, 8 rows 34 / 37 and 43 /
+// 46, hidden 2048 10 rows 48 / 53 and 60 / 64; 4 of 4 8 rows 30 / 39 and 46 /
+// 48, 10 rows 34 / 39 and 57 / 48; 4 of 1, hidden 512, 10 rows 32 / 36 and 39 /
+// 43, hidden 2048 14 rows 46 / 51 and 54 / 59; 2 of 1, hidden 512, 12 rows 32 /
+// 34 and 38 / 42, hidden 2048 16 rows 46 / 49 and 52 / 56; 4 of 2, hidden 4096
+// (the four launches' projection is slower there), 12 rows 94 / 79.
 constexpr int kPromptMinTokens = 8;
+static int prompt_min_tokens(int heads, int kvh, int hidden) {
+  const int size = heads + 2 * kvh;
+  const bool mid = hidden > 1024 && hidden <= 2048;
+  if (size >= 16) return kPromptMinTokens;
+  if (size >= 10) return mid ? 12 : 10;
+  if (size >= 6) return mid ? 16 : 12;
+  return mid ? 18 : 14;
+}
 
 struct AttnArgs {
   const float* qg;      // [T, heads * 2 * hd] projected query/gate pairs
@@ -1776,7 +1793,8 @@ int fk_attention_decode(const void* hidden, int hidden_dtype, const void* norm_w
       return check_launch("attn_step_kernel");
     }
   }
-  if (tokens >= kPromptMinTokens && attn_prompt_ok(tokens, hidden_size, heads, kv_heads, head_dim, weight_dtype, norm_dtype))
+  if (tokens >= prompt_min_tokens(heads, kv_heads, hidden_size) &&
+      attn_prompt_ok(tokens, hidden_size, heads, kv_heads, head_dim, weight_dtype, norm_dtype))
     return launch_attn_prompt(call, ws.prompt, s);
   st = fk_attention_project(hidden, hidden_dtype, norm_weight, norm_dtype, q_proj, k_proj, v_proj, weight_dtype,
                             tokens, hidden_size, 2 * heads * head_dim, kv_heads * head_dim, eps, 1.0f, ws.qg, ws.k,

@@ -66,6 +66,12 @@ def _reference(x, kc, vc, w, start, heads, kvh, rope_dim, theta, interleaved):
     (65, 15, 1024, 4, 4, torch.bfloat16, torch.bfloat16, True),
     (200, 1000, 2048, 16, 2, torch.float32, torch.float32, True),
     (131, 777, 512, 8, 4, torch.float32, torch.bfloat16, False),
+    # either side of the decode entry's line for few heads
+    (9, 40, 512, 8, 1, torch.float32, torch.float32, True),
+    (10, 40, 512, 8, 1, torch.float32, torch.float32, True),
+    (17, 200, 2048, 2, 1, torch.bfloat16, torch.float32, True),
+    (18, 200, 2048, 2, 1, torch.bfloat16, torch.float32, True),
+    (8, 21, 1536, 12, 3, torch.float32, torch.bfloat16, True),
 ])
 def test_prompt_rows(tokens, start, hidden, heads, kvh, x_dtype, cache_dtype, interleaved):
     x, kc, vc, w = _inputs(tokens, tokens, hidden, heads, kvh, start + tokens + 3, x_dtype, cache_dtype)
@@ -246,12 +252,12 @@ def test_infinite_value_of_the_call_stays_infinite(tokens, start, row):
     """One value of one row overflows: the rows that see it get that infinity,
     in that dim alone, and the rows before it nothing."""
 
-    x, kc, vc, w = _inputs(4, tokens, 512, 8, 2, start + tokens, torch.float32, torch.float32)
+    x, kc, vc, w = _inputs(4, tokens, 512, 16, 2, start + tokens, torch.float32, torch.float32)
     x[:, 3], x[row, 3] = 0.0, 5.0
     w["norm_weight"][3] = 0.0
     w["v_proj_weight"][5], w["v_proj_weight"][5, 3] = 0.0, 3e38  # kv head 0, dim 5
-    w["out_proj_weight"][:, 5:4 * 256:256] = 0.02               # of its four query heads: the infinities add up
-    kw = dict(start_position=start, attention_heads=8, kv_heads=2, rope_dim=64)
+    w["out_proj_weight"][:, 5:8 * 256:256] = 0.02               # of its eight query heads: the infinities add up
+    kw = dict(start_position=start, attention_heads=16, kv_heads=2, rope_dim=64)
     got, _, v = hip.hip_qwen36_batched_attention_decode(x, kc, vc, *w.values(), **kw)
     assert bool(v[start + row, 0, 5].isposinf()) and int((~v.isfinite()).sum()) == 1
     assert bool(got[row:].isposinf().all())
