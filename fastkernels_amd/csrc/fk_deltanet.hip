@@ -292,7 +292,10 @@ struct ConvArgs {
 // workgroups (0.39 us a row: 198 us at 512 rows, 8,192 channels; in blocks of
 // 8 rows 12).  Outputs written over the inputs (or the state in place) keep
 // one block of all rows, where a thread reads what it overwrites first.
+// (NT: rows loaded at once; a call of one row takes 3.7 us with 1, as before the
+// blocks, and 3.9 with 8.)
 constexpr int kConvTokens = 8;
+template <int NT>
 __global__ __launch_bounds__(256) void deltanet_conv_kernel(ConvArgs a) {
   const int c = blockIdx.x * 256 + threadIdx.x;
   if (c >= a.C) return;
@@ -307,13 +310,13 @@ __global__ __launch_bounds__(256) void deltanet_conv_kernel(ConvArgs a) {
                        : load_scalar(a.mixed, a.mixed_dt, (size_t)u * a.C + c);
     wk[j] = j < a.KS ? load_scalar(a.w, a.w_dt, (size_t)c * a.KS + j) : 0.f;
   }
-  for (int tb = t0; tb < t1; tb += kConvTokens) {
-    float in[kConvTokens];
+  for (int tb = t0; tb < t1; tb += NT) {
+    float in[NT];
 #pragma unroll
-    for (int i = 0; i < kConvTokens; ++i)
+    for (int i = 0; i < NT; ++i)
       in[i] = load_scalar(a.mixed, a.mixed_dt, (size_t)min(tb + i, t1 - 1) * a.C + c);
 #pragma unroll
-    for (int i = 0; i < kConvTokens; ++i) {
+    for (int i = 0; i < NT; ++i) {
       if (tb + i >= t1) break;
 #pragma unroll
       for (int j = 0; j < 7; ++j)
@@ -345,7 +348,8 @@ static int launch_conv(ConvArgs ca, hipStream_t s) {
                         ranges_overlap(ca.state, ns, ca.next_state, ns);
   ca.rows = in_place ? ca.T : kConvTokens;
   const dim3 grid((unsigned)((ca.C + 255) / 256), (unsigned)((ca.T + ca.rows - 1) / ca.rows));
-  hipLaunchKernelGGL(deltanet_conv_kernel, grid, dim3(256), 0, s, ca);
+  if (ca.T == 1) hipLaunchKernelGGL(deltanet_conv_kernel<1>, grid, dim3(256), 0, s, ca);
+  else hipLaunchKernelGGL(deltanet_conv_kernel<kConvTokens>, grid, dim3(256), 0, s, ca);
   return check_launch("deltanet_conv_kernel");
 }
 
