@@ -346,7 +346,8 @@ static int launch_conv(ConvArgs ca, hipStream_t s) {
   const size_t n = (size_t)ca.T * ca.C, ns = (size_t)ca.C * ca.KS * (ca.state_dt == FK_DTYPE_BF16 ? 2 : 4);
   const bool in_place = ranges_overlap(ca.mixed, n * (ca.mixed_dt == FK_DTYPE_BF16 ? 2 : 4), ca.out, n * 4) ||
                         ranges_overlap(ca.state, ns, ca.next_state, ns);
-  ca.rows = in_place ? ca.T : kConvTokens;
+  // (blocks of 8 rows, of more past the 65,535 of them that a grid's second dimension holds)
+  ca.rows = in_place ? ca.T : (ca.T / 65535 / kConvTokens + 1) * kConvTokens;
   const dim3 grid((unsigned)((ca.C + 255) / 256), (unsigned)((ca.T + ca.rows - 1) / ca.rows));
   if (ca.T == 1) hipLaunchKernelGGL(deltanet_conv_kernel<1>, grid, dim3(256), 0, s, ca);
   else hipLaunchKernelGGL(deltanet_conv_kernel<kConvTokens>, grid, dim3(256), 0, s, ca);

@@ -45,6 +45,18 @@ def test_conv_blocks(tokens, kernel_size):
     assert torch.equal(nxt.cpu(), comb[:, -kernel_size:])
 
 
+def test_conv_of_more_blocks_than_a_grid_dimension_holds():
+    """524,281 rows and more are over 65,535 blocks of 8: the blocks grow."""
+
+    gen = torch.Generator().manual_seed(6)
+    mixed, state, w = _randn(gen, (524_300, 3)), _randn(gen, (3, 4)), _randn(gen, (3, 1, 4))
+    out, nxt = hip.hip_qwen36_batched_deltanet_conv(mixed.cuda(), state.cuda(), w.cuda())
+    comb = torch.cat((state, mixed.t()), dim=1)
+    ref = F.silu(F.conv1d(comb.double()[None, :, 1:], w.double(), groups=3)[0]).t()
+    assert torch.allclose(out.cpu().double(), ref, rtol=1e-5, atol=4 * 25 * 2.0 ** -23)
+    assert torch.equal(nxt.cpu(), comb[:, -4:])
+
+
 @pytest.mark.parametrize("tokens,qk_heads,value_heads,head_dim", [
     (2, 16, 32, 128), (3, 16, 32, 128), (15, 2, 4, 128), (16, 4, 4, 128), (17, 16, 32, 128), (32, 1, 2, 128), (51, 16, 32, 128),
     (19, 2, 4, 64), (95, 2, 4, 128), (96, 1, 5, 128), (97, 2, 4, 128), (112, 16, 32, 128), (127, 1, 2, 128), (100, 4, 4, 128),
