@@ -53,6 +53,9 @@ int main() {
       sink += fk_moe_workspace_bytes(16, a, 256, b, 2048);
       sink += fk_attention_workspace_bytes(a, b, 2, 256);
       sink += fk_attention_workspace_bytes(1, 16, a, b);
+      sink += fk_attention_prompt_workspace_bytes(a, b, 16, 2, 256, 1, 1);
+      sink += fk_attention_prompt_workspace_bytes(a, 2048, b, 2, 256, 1, 1);
+      sink += fk_attention_prompt_workspace_bytes(64, 2048, a, b, 256, 1, 1);
       sink += fk_deltanet_workspace_bytes(a, b, 128);
       sink += fk_deltanet_step_workspace_bytes(a, 16, b, 128);
       sink += fk_deltanet_step_workspace_bytes(8, a, 32, b);
@@ -150,6 +153,21 @@ int main() {
                                      256, -1, 1e7f, 1, 1e-6f, 1e-6f, fp, fp, p, sizeof(buf), nullptr));
   EXPECT_REFUSED(fk_attention_decode(p, 1, p, 1, p, p, p, p, 1, p, p, 1, p, p, 0, 1024, 0, nullptr, 1, 2048, 16, 2,
                                      256, 64, 1e7f, 1, 1e-6f, 1e-6f, fp, fp, p, 64, nullptr));
+  EXPECT_REFUSED(fk_attention_decode(p, 1, p, 1, p, p, p, p, 1, p, p, 1, p, p, 0, 1024, 2147483647, nullptr, 8, 2048, 16,
+                                     2, 256, 64, 1e7f, 1, 1e-6f, 1e-6f, fp, fp, p, sizeof(buf), nullptr));
+  EXPECT_REFUSED(fk_attention_prompt(nullptr, 1, nullptr, 1, nullptr, nullptr, nullptr, nullptr, 1, nullptr, nullptr, 1,
+                                     nullptr, nullptr, 0, 1024, 0, 40, 2048, 16, 2, 256, 64, 1e7f, 1, 1e-6f, 1e-6f,
+                                     nullptr, nullptr, nullptr, 0, nullptr));
+  EXPECT_REFUSED(fk_attention_prompt(p, 1, p, 1, p, p, p, p, 1, p, p, 1, p, p, 0, 1024, 0, 0, 2048, 16, 2, 256, 64,
+                                     1e7f, 1, 1e-6f, 1e-6f, fp, fp, p, sizeof(buf), nullptr));
+  EXPECT_REFUSED(fk_attention_prompt(p, 1, p, 1, p, p, p, p, 1, p, p, 1, p, p, 0, 1024, 2147483647, 40, 2048, 16, 2, 256,
+                                     64, 1e7f, 1, 1e-6f, 1e-6f, fp, fp, p, sizeof(buf), nullptr));
+  EXPECT_REFUSED(fk_attention_prompt(p, 1, p, 1, p, p, p, p, 1, p, p, 1, p, p, 0, 1024, 0, 40, 2048, 32, 2, 256, 64,
+                                     1e7f, 1, 1e-6f, 1e-6f, fp, fp, p, sizeof(buf), nullptr));
+  EXPECT_REFUSED(fk_attention_prompt(p, 1, mis, 1, p, p, p, p, 1, p, p, 1, p, p, 0, 1024, 0, 40, 2048, 16, 2, 256, 64,
+                                     1e7f, 1, 1e-6f, 1e-6f, fp, fp, p, sizeof(buf), nullptr));
+  EXPECT_REFUSED(fk_attention_prompt(p, 1, p, 1, p, p, p, p, 1, p, p, 1, p, p, 0, 1024, 0, 40, 2048, 16, 2, 256, 64,
+                                     1e7f, 1, 1e-6f, 1e-6f, fp, fp, p, sizeof(buf), nullptr));
 
   // DeltaNet
   EXPECT_REFUSED(fk_deltanet_project(nullptr, 1, nullptr, 1, nullptr, nullptr, nullptr, nullptr, 1, 1, 2048, 8192, 4096,

@@ -185,6 +185,42 @@ def test_entry_points_reject_bad_arguments_before_launch():
     assert st == _lib.FK_ERR_INVALID
 
 
+def test_attention_prompt_refuses_what_it_does_not_take():
+    lib = _lib.load()
+    store = (ctypes.c_uint8 * 256)()
+    p = ctypes.addressof(store) + (-ctypes.addressof(store) % 16)  # aligned, never read by a refused call
+    base = dict(hidden=p, x_dt=0, norm=p, n_dt=1, wq=p, wk=p, wv=p, wo=p, w_dt=1, qn=p, kn=p, qk_dt=1, kc=p, vc=p, c_dt=0,
+                positions=1024, start=0, tokens=40, hidden_size=2048, heads=16, kv_heads=2, head_dim=256, rope=64, theta=1e4,
+                interleaved=1, eps=1e-6, qk_eps=1e-6, update=p, out=None, ws=p, ws_bytes=1 << 40, stream=None)
+
+    def refused(status, message, **change):
+        assert _err("fk_attention_prompt", *{**base, **change}.values()) == status, change
+        assert message in lib.fk_last_error_detail(), (change, lib.fk_last_error_detail())
+
+    refused(_lib.FK_ERR_INVALID, b"tokens", tokens=0)
+    refused(_lib.FK_ERR_INVALID, b"rope_dim", rope=-1)
+    refused(_lib.FK_ERR_INVALID, b"even rope_dim", rope=7, interleaved=0)
+    for change in (dict(start=-1), dict(start=985), dict(start=(1 << 31) - 1), dict(positions=0)):
+        refused(_lib.FK_ERR_INVALID, b"exceed the cache length", **change)
+    for name in ("x_dt", "qk_dt", "c_dt"):
+        refused(_lib.FK_ERR_DTYPE, b"f32 or bf16", **{name: 9})
+    # the shapes whose workspace is 0 bytes: head_dim, groups of query heads, more than 4,096 query values, hidden
+    # sizes off the K step, weights and norms that are not bf16
+    for change in (dict(head_dim=128), dict(heads=16, kv_heads=3), dict(heads=16, kv_heads=1), dict(heads=6, kv_heads=2),
+                   dict(heads=32, kv_heads=4), dict(hidden_size=2040), dict(w_dt=0), dict(n_dt=0)):
+        refused(_lib.FK_ERR_UNSUPPORTED, b"fk_attention_decode", **change)
+        a = {**base, **change}
+        assert lib.fk_attention_prompt_workspace_bytes(*(a[k] for k in (
+            "tokens", "hidden_size", "heads", "kv_heads", "head_dim", "w_dt", "n_dt"))) == 0, change
+    for name in ("hidden", "norm", "wq", "wk", "wv", "wo", "qn", "kn", "kc", "vc", "update"):
+        refused(_lib.FK_ERR_INVALID, b"non-NULL", **{name: None})
+    for name in ("hidden", "norm", "wq", "wk", "wv", "wo", "kc", "vc", "ws"):
+        refused(_lib.FK_ERR_ALIGNMENT, b"16-byte aligned", **{name: p + 8})
+    refused(_lib.FK_ERR_WORKSPACE, b"workspace needs", ws=None)
+    refused(_lib.FK_ERR_WORKSPACE, b"workspace needs",
+            ws_bytes=lib.fk_attention_prompt_workspace_bytes(40, 2048, 16, 2, 256, 1, 1) - 1)
+
+
 def test_workspace_too_small_is_reported():
     buf = (ctypes.c_uint8 * 64)()
     addr = ctypes.addressof(buf)

@@ -57,6 +57,39 @@ def test_conv_of_more_blocks_than_a_grid_dimension_holds():
     assert torch.equal(nxt.cpu(), comb[:, -4:])
 
 
+@pytest.mark.parametrize("state_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("tokens", [3, 20, 97, 128])
+def test_recurrence_in_place_and_bf16_states(tokens, state_dtype):
+    """The C entry with the next state over the state, of either type (the scan
+    and the chunks), and with outputs off the 16-byte boundary, gives what
+    separate ones give; a bf16 state is read exactly and rounds once."""
+
+    from fastkernels_amd import _lib
+
+    gen = torch.Generator().manual_seed(tokens)
+    mixed, z = _randn(gen, (tokens, 2 * 2 * 128 + 512)).cuda(), _randn(gen, (tokens, 512)).cuda()
+    a, b = _randn(gen, (tokens, 4)).cuda(), _randn(gen, (tokens, 4)).cuda()
+    state = _randn(gen, (4, 128, 128), 0.1).to(state_dtype).cuda()
+    rest = [_randn(gen, (256, 512), 0.02, torch.bfloat16).cuda(), *(_randn(gen, s).cuda() for s in ((128,), (4,), (4,)))]
+    run = lambda s: hip.hip_qwen36_batched_deltanet_recurrent_output(  # noqa: E731
+        mixed, z, a, b, s, *rest, qk_heads=2, value_heads=4, head_dim=128)
+    update, after = run(state)
+    update32, after32 = run(state.float())
+    assert after.dtype == state_dtype and torch.equal(update, update32) and torch.equal(after, after32.to(state_dtype))
+    import ctypes
+    codes = (ctypes.c_int32 * 10)(0, 0, 0, 0, 0 if state_dtype == torch.float32 else 1, 1, 0, 0, 0, 0)
+    n = _lib.load().fk_deltanet_workspace_bytes(tokens, 4, 128)
+    ws = torch.zeros(n, dtype=torch.uint8, device="cuda")
+    store = torch.zeros(2 * tokens * 256 + 8, device="cuda")
+    residual = _randn(gen, (tokens, 256)).cuda()
+    got, out = store[1:1 + tokens * 256], store[3 + tokens * 256:3 + 2 * tokens * 256]  # 4 and 12 bytes past a boundary
+    _lib.call("fk_deltanet_recurrent_output", *(t.data_ptr() for t in (mixed, z, a, b, state, *rest, residual)),
+              ctypes.cast(codes, ctypes.c_void_p), tokens, 2, 4, 128, 256, 1e-6, got.data_ptr(), state.data_ptr(),
+              out.data_ptr(), ws.data_ptr(), n, torch.cuda.current_stream().cuda_stream)
+    assert torch.equal(got.view(tokens, 256), update) and torch.equal(state, after)
+    assert torch.equal(out.view(tokens, 256), residual + update)
+
+
 @pytest.mark.parametrize("tokens,qk_heads,value_heads,head_dim", [
     (2, 16, 32, 128), (3, 16, 32, 128), (15, 2, 4, 128), (16, 4, 4, 128), (17, 16, 32, 128), (32, 1, 2, 128), (51, 16, 32, 128),
     (19, 2, 4, 64), (95, 2, 4, 128), (96, 1, 5, 128), (97, 2, 4, 128), (112, 16, 32, 128), (127, 1, 2, 128), (100, 4, 4, 128),

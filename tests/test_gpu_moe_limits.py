@@ -5,9 +5,12 @@ The reference router accepts hidden sizes up to 4096 and up to 1024 experts
 intermediate sizes up to 1024 (qwen36_expert.py:850-851); the HIP entry
 points accept the same.  These shapes reach kernels the model's own shapes
 never run:
-  * the grid-barrier router (moe_router_kernel) for more than 256 experts,
-    hidden sizes above 2048 or more than 256 tokens, with 64-bit top-k keys
-    from 512 experts on;
+  * the routers of more than 256 experts, hidden sizes above 2048 or more
+    than 256 tokens: the grid-barrier kernel (moe_router_kernel), with 64-bit
+    top-k keys from 512 experts on, for a few tokens, fp32 router or norm
+    weights, experts that are no multiple of 16 and hidden sizes that are none
+    of 64; else logits on the matrix cores with moe_topk_kernel and
+    moe_align_kernel after them;
   * the gate/up GEMV with eight 8-element chunks per lane (H > 2048);
   * the down GEMV with two chunks per lane (I > 512);
   * hidden sizes that are multiples of 8 but not of 16 (odd chunk counts),
@@ -71,6 +74,7 @@ def _check(device, e, h, i, tokens, seed):
     "e,h,i,tokens",
     [
         (512, 1024, 128, 4),    # > 256 experts: grid-barrier router, 64-bit keys
+        (512, 1024, 128, 17),   # past its line: logits on the matrix cores
         (1024, 512, 64, 3),     # the expert limit
         (64, 3072, 128, 5),     # H > 2048: 8 chunks per lane in router and gate/up
         (16, 4096, 1024, 2),    # the hidden and intermediate limits together
@@ -84,9 +88,43 @@ def test_moe_layer_at_operator_limits(device, e, h, i, tokens):
 
 @pytest.mark.parametrize("e,h,i,tokens", [(64, 512, 64, 257), (64, 512, 256, 512)])
 def test_moe_layer_beyond_256_tokens(device, e, h, i, tokens):
-    # grid-barrier router for T > 256; GEMV experts (I = 64) and MFMA experts
+    # the matrix-core router for T > 256; GEMV experts (I = 64) and MFMA experts
     # (I = 256) after it; T * K = 4096 is the routing-table limit
     _check(device, e, h, i, tokens, seed=200 + tokens + i)
+
+
+# what the matrix-core router does not take: an fp32 router weight or norm
+# weight, experts no multiple of 16, a hidden size no multiple of 64
+@pytest.mark.parametrize("e,h,tokens,what", [
+    (64, 512, 257, "router"),
+    (256, 1024, 512, "router"),
+    (512, 512, 65, "router"),
+    (1024, 256, 20, "norm"),
+    (1024, 512, 512, "norm"),
+    (250, 512, 300, "experts"),
+    (40, 3080, 9, "hidden"),
+    (48, 3080, 257, "hidden"),
+])
+def test_grid_barrier_router(device, e, h, tokens, what):
+    print(f"grid-barrier router E={e} H={h} T={tokens} {what}", flush=True)
+    norm, router = _weights(e, h, 8, seed=500 + e + tokens)[:2]
+    if what == "router":
+        router = router.float()
+    if what == "norm":
+        norm = norm.float()
+    x = wl.make_hidden(tokens, h, seed=501)
+    logits, ids, wt = hip.hip_qwen36_batched_moe_router_decode(x.to(device), norm.to(device), router.to(device), top_k=K)
+    o_logits, _, _ = oracle.router(x, norm, router, K)
+    torch.testing.assert_close(logits.cpu(), o_logits, atol=1e-4, rtol=1e-4)
+    assert_routing_parity(logits, ids, wt, o_logits, K)
+    hip.workspace_status(device)
+    # the experts read the tables that this kernel's last workgroup built
+    if what == "router" and e == 64:
+        w = _weights(e, h, 64, seed=502)
+        args = (norm, router, *w[2:])
+        _, moe, _, l_ids, l_wt = hip.hip_qwen36_batched_moe_layer_decode(x.to(device), *(t.to(device) for t in args), top_k=K)
+        ref = oracle.routed_experts(x, l_ids.cpu(), l_wt.cpu(), w[2], w[3]) + oracle.shared_expert(x, w[4], w[5], w[6])
+        torch.testing.assert_close(moe.cpu(), ref, **tol(torch.bfloat16))
 
 
 @pytest.mark.parametrize(

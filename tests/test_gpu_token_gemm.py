@@ -96,3 +96,20 @@ def test_values_past_the_bf16_range(tokens):
     w = [_randn(gen, (n, 512), 0.02) for n in (64, 32, 16, 16)]
     for out in hip.hip_qwen36_batched_deltanet_project(x, norm, *w):
         assert bool((out[2:4] == 0).all()) and bool(out.isfinite().all())
+
+
+@pytest.mark.parametrize("tokens", [13, 70, 300])
+def test_outputs_off_the_16_byte_boundary(tokens):
+    """The C entry's outputs need no alignment: the same values one float at a time."""
+
+    from fastkernels_amd import _lib
+
+    gen = torch.Generator().manual_seed(tokens)
+    x, norm = _randn(gen, (tokens, 512), 1.0, torch.float32), _randn(gen, (512,), 0.1)
+    w = [_randn(gen, (n, 512), 0.02) for n in (4096, 512, 512)]
+    want = hip.hip_qwen36_batched_attention_project(x, norm, *w)
+    stores = [torch.full((tokens * n.shape[0] + 2,), 7.0, device="cuda") for n in w]
+    _lib.call("fk_attention_project", x.data_ptr(), 0, norm.data_ptr(), 1, *(t.data_ptr() for t in w), 1, tokens, 512, 4096,
+              512, 1e-6, 1.0, *(t[1:].data_ptr() for t in stores), torch.cuda.current_stream().cuda_stream)
+    for store, o in zip(stores, want):
+        assert torch.equal(store[1:-1].view_as(o), o) and float(store[0]) == 7.0 and float(store[-1]) == 7.0

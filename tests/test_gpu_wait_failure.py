@@ -80,12 +80,15 @@ def _exercise(plan):
         assert torch.equal(a, b)
 
 
-@pytest.mark.parametrize("tokens", [1, 16, 300])
-def test_moe_layer_wait_failure_is_poisoned_and_flagged(device, small_moe, tokens):
+@pytest.mark.parametrize("tokens,router", [(1, torch.bfloat16), (16, torch.bfloat16), (300, torch.bfloat16),
+                                           (300, torch.float32)])
+def test_moe_layer_wait_failure_is_poisoned_and_flagged(device, small_moe, tokens, router):
     # T = 1: single-launch layer; T = 16: tagged router + GEMV experts;
-    # T = 300: grid-barrier router + MFMA experts
-    print(f"moe wait failure tokens={tokens}", flush=True)
-    plan = MoeLayerPlan(small_moe, tokens)
+    # T = 300: MFMA experts after the matrix-core router, whose selection waits
+    # for nothing but heeds the bound and the flag, and (fp32 router weights)
+    # after the grid-barrier router
+    print(f"moe wait failure tokens={tokens} router={router}", flush=True)
+    plan = MoeLayerPlan({**small_moe, "router_weight": small_moe["router_weight"].to(router)}, tokens)
     plan.hidden.copy_(wl.make_hidden(tokens, SMALL.hidden_size, seed=33).to(device))
     _exercise(plan)
 
