@@ -15,18 +15,21 @@
 // Tile: BN weight rows x BM tokens per workgroup, K in steps of 64.  Both
 // operands go through LDS in 128-byte rows whose 16-byte chunks are
 // XOR-swizzled by the row (chunk ^ (row & 7)): the row-wise staging writes and
-// the operand reads (16 rows x 16 B) measured no bank conflicts.  Weight and
+// the operand reads (16 rows x 16 B) show no bank conflicts in the counters.  Weight and
 // token loads are one to four steps ahead of the step that computes.
+//
+// An infinite weight makes its row NaN (an infinity times the terms' signs and
+// zeros), a token's infinity its own products infinite or NaN as fp32 ones.
 //
 // What bounds it: at a few dozen tokens the latency of a step (LDS write,
 // barrier, LDS read, a chain of six MFMAs: ~0.7 us with one workgroup on a
 // CU), which double-buffered LDS, eight wavefronts and small tiles shorten; at
 // hundreds of tokens the MFMAs with the fp32 -> bf16 split beside them, which
-// large tiles amortise (780-880 of the 1206 TFLOP/s a library bf16 GEMM
-// reaches, three MFMAs per product counted).  The DeltaNet input projections
-// (12,352 rows, K 2048) before (VALU, whole rows per wavefront) and now, us:
-// 8 tokens 41.6 / 26.5, 32 110 / 28, 64 201 / 32, 128 388 / 42, 256 829 / 64,
-// 512 2062 / 100, 1000 4011 / 195.
+// large tiles amortise (770 of the 1206 TFLOP/s a library bf16 GEMM reaches,
+// three MFMAs per product counted; under a profiler 40 to 46% of the busy CUs'
+// matrix cycles).  The DeltaNet input projections (12,352 rows, K 2048), VALU
+// kernel (whole rows per wavefront) / here, us: 8 tokens 38 / 25.5, 32 105 / 26,
+// 64 197 / 31, 128 385 / 41, 256 796 / 64, 512 2056 / 101, 1000 4006 / 198.
 #include "fk_common.h"
 #include "fk_host.h"
 
@@ -378,15 +381,17 @@ static void launch_tile(int tile, const GemmArgs& a, hipStream_t s) {
 }
 
 // Measured time of a tile's workgroups over K = 2048, us: one round of at
-// most one workgroup per CU, and each further round (12,352 rows, 16 to 1000
-// tokens; further rounds of the small tiles share CUs).  The tile with the
-// smallest estimate is taken: small tiles while one round of them holds the
-// batch, large ones where the split of the tokens would be redone often.
+// most one workgroup per CU, and each further round (12,352 and 9,216 rows, 16
+// to 1024 tokens, every tile at every size; further rounds of the small tiles
+// share CUs).  The tile with the smallest estimate is taken: small tiles while
+// one round of them holds the batch, large ones where the split of the tokens
+// would be redone often (within 2% of the best tile on average, 11% at worst:
+// 105 for 93 at 257 to 320 tokens of 12,352 rows).
 struct GemmTile {
   int bn, bm;
   float first, next;
 };
-constexpr GemmTile kGemmTiles[] = {{64, 32, 24.f, 12.f}, {64, 64, 30.f, 20.f}, {128, 64, 40.f, 28.f}, {128, 128, 50.f, 53.f}, {256, 128, 86.f, 90.f}};
+constexpr GemmTile kGemmTiles[] = {{64, 32, 26.f, 13.f}, {64, 64, 31.5f, 19.f}, {128, 64, 39.f, 34.f}, {128, 128, 57.f, 58.f}, {256, 128, 90.f, 97.f}};
 
 static int pick_tile(int T, int R, int splits) {
   const int cus = device_cus() > 0 ? device_cus() : 256;
