@@ -15,8 +15,8 @@
 //
 // Kernels: T <= 4 at the shapes attn_step_chunks accepts (the model's) run
 // as one launch, attn_step_kernel (below); prompt_min_tokens rows or more at
-// the shapes attn_prompt_ok accepts as matrix products (fk_attention_prompt.hip); other
-// steps as four launches:
+// the shapes attn_prompt_ok accepts as matrix products
+// (fk_attention_prompt.hip); other steps as four launches:
 //   attn_proj_kernel  RMSNorm folded into a GEMV over [Wq | Wk | Wv] (9216
 //                     rows at the model shape); H > 2048 takes the shared
 //                     normalized projection kernel of fk_deltanet.hip
@@ -712,9 +712,9 @@ constexpr int kAsTile = 24;        // cached positions per LDS tile of an attent
 // Chunks of more positions than this (a third tile for the loop over tiles,
 // which waits for its cached rows once per tile past the first) take the
 // pipelined MFMA softmax.  Both sides, us per step, bf16 cache and hidden
-// 2048: chunks of 40 positions 24.75 by tiles, 24.75 by MFMA; 44 (4 tokens)
-// 33.1 and 33.8; 52 26.4 and 25.0; 57 (4 tokens) 34.5 and 33.2; 188 35.8 and
-// 30.5; 750 (4 tokens) 86.1 and 59.3.
+// 2048: chunks of 40 positions 24.1 by tiles, 24.3 by MFMA; 48 24.4 and 24.8 (4
+// tokens 33.1 and 33.5); 49 25.7 and 24.7 (4 tokens 34.5 and 33.6); 57 26.4
+// and 25.3; 188 36.8 and 31.7; 751 (4 tokens) 89 and 63.
 constexpr int kAsLongMin = 2 * kAsTile;
 constexpr int kAsMaxH = 2048;
 constexpr int kAsMaxG = 8;         // query heads per kv head

@@ -14,8 +14,8 @@
 //
 // Calls of 32 rows (four launches, each streaming every weight, with VALU
 // dot products) took 1417 us for 200 rows behind 1,000 positions and 2650 for
-// 256 behind 3,000; this takes 178 and 249.  The rows' own keys and values enter unrounded for every row of the
-// call, whatever the cache's type.
+// 256 behind 3,000; this takes 179 to 187 and 265.  The rows' own keys and
+// values enter unrounded for every row of the call, whatever the cache's type.
 #include "fk_common.h"
 #include "fk_host.h"
 
@@ -25,9 +25,9 @@ constexpr int kPromptHd = 256;    // head_dim
 constexpr int kPromptRows = 64;   // query rows (token, head of one kv head) per workgroup, 16 per wavefront
 constexpr int kPromptTile = 16;   // positions per tile
 // Workgroups aimed at when the positions are split into chunks: two per CU.
-// (384 / 512 / 1024, us a call: 256 rows behind 3,000 positions 287 / 249 /
-// 263, 200 behind 1,000 170 / 178 / 172, 64 behind 3,000 115 / 115 / 130: more
-// chunks cost the merge.)
+// (384 / 512 / 1024, us a call: 256 rows behind 3,000 positions 302 / 266 /
+// 276, 200 behind 1,000 174 / 186 / 174, 64 behind 3,000 122 / 118 / 135, 32
+// behind 3,000 99 / 102 / 102: more chunks cost the merge.)
 constexpr int kPromptWgs = 512;
 constexpr int kPromptMaxChunks = 64;
 

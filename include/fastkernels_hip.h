@@ -263,8 +263,9 @@ size_t fk_attention_workspace_bytes(int tokens, int heads, int kv_heads, int hea
  * 8 (a multiple of 4 above 4) and heads * head_dim a multiple of 512 (the
  * model's shapes) this is one launch whose workgroups hand values to each
  * other (the workspace then also carries the error word of
- * fk_workspace_status); more tokens at the shapes fk_attention_prompt takes run
- * its kernels, other calls four launches.
+ * fk_workspace_status); from 8 tokens (more with fewer than 16 query heads and
+ * few kv heads) the shapes fk_attention_prompt takes run its kernels, other
+ * calls four launches.
  * Replaces triton_qwen36_batched_attention_decode (qwen36_attention.py:448-577)
  * and the residual add of triton_qwen36_batched_attention_moe_layer_decode
  * (qwen36_layer.py:109-201). */
@@ -282,8 +283,11 @@ int fk_attention_decode(const void* hidden, int hidden_dtype,
                         void* workspace, size_t workspace_bytes, void* stream);
 
 /* Bytes of workspace for fk_attention_prompt, or 0 for a shape it does not
- * take (head_dim 256, heads / kv_heads a power of two up to 8, bf16 weights
- * and norm weight, hidden_size a multiple of 64). */
+ * take (head_dim 256, heads / kv_heads a power of two up to 8, heads * 256 <=
+ * 4096, kv_heads <= 64, bf16 weights and norm weight, hidden_size a multiple of
+ * 64).  Never less for more tokens; about 90 KB a row at the model's shape, so
+ * a caller splits long prompts into calls (of 1,024 rows, the fastest measured;
+ * rows of an earlier call are read back from the caches). */
 size_t fk_attention_prompt_workspace_bytes(int tokens, int hidden_size, int heads, int kv_heads, int head_dim,
                                            int weight_dtype, int norm_dtype);
 
@@ -330,7 +334,8 @@ int fk_deltanet_conv(const void* mixed, int mixed_dtype,
                      int tokens, int channels, int kernel_size,
                      float* conv_out, void* next_state, void* stream);
 
-/* Bytes of workspace for fk_deltanet_recurrent_output. */
+/* Bytes of workspace for fk_deltanet_recurrent_output; never less for more
+ * tokens. */
 size_t fk_deltanet_workspace_bytes(int tokens, int value_heads, int head_dim);
 
 /* Gated delta rule over `tokens` consecutive rows through one recurrent
